@@ -144,7 +144,11 @@ Layout make_layout(const MxModel& m) {
     L.win = kWindowWords;
     if (rows && (m.nmesh > 0 || !m.boxbox_primitive)) {
       int it = m.epa_iterations > 0 ? m.epa_iterations : 0;
-      L.epa_vc = 10 + 2 * it;
+      // five vertices at most to start with and one more per expansion step.  (At the reference's
+      // 10 + 2 it vertices the dense-clutter scene's window took 2792 words and a CU held fifteen
+      // worlds; at 2480 it holds sixteen, and 8192 worlds are two full rounds instead of two and an
+      // almost empty third.)
+      L.epa_vc = 6 + it;
       L.epa_fc = 6 + 5 * it;
       int poly = round_up(cvx::poly_words(L.epa_vc, L.epa_fc), 4), need = poly + kEpaRequest + cvx::kManifoldWords;
 #ifdef MX_SLAB
@@ -199,23 +203,28 @@ Layout make_layout(const MxModel& m) {
   // then the hull vertices (4 words each), read by every support-point search of the stage
   L.meshw = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
   if (m.njmax > 0 && m.nmeshvert > 0 && L.win < L.meshw + 4 * m.nmeshvert) L.win = round_up(L.meshw + 4 * m.nmeshvert, 4);
-  // row-group EPA: four (else two) blocks of a small polytope, its request / result words and a
-  // box-manifold clip block, side by side at the start of the window, when they and the collision
-  // records after them fit the window as sized above (the blocks never grow the window)
+  // The EPA region before the collision records grows, as far as the window as sized above has room,
+  // for what shares it: first the contact staging of collide() (a pair table of kStagePair words per
+  // lane and kStageContact words per contact of a candidate batch; the region is dead once the
+  // batch's EPA ends), then row-group EPA (four, else three or two blocks of a small polytope, its
+  // request / result words and a box-manifold clip block, side by side).
   L.epa_ng = 0;
+  L.stage = -1;
   if (m.njmax > 0 && L.epa == 0) {
+    auto region = [&](int words) {   // whether the region can take so many words; it does then
+      const int at = words > L.gpose ? words : L.gpose, meshw = round_up(at + GP_WORDS * m.ngeom, 4);
+      if (meshw + 4 * m.nmeshvert > L.win) return false;
+      L.gpose = at;
+      L.meshw = meshw;
+      return true;
+    };
+    if (region(kStagePair * kLanes + kStageContact * m.nconmax)) L.stage = 0;
     L.epa_svc = kSmallPolyVerts < L.epa_vc ? kSmallPolyVerts : L.epa_vc;
     L.epa_sfc = kSmallPolyFaces < L.epa_fc ? kSmallPolyFaces : L.epa_fc;
     L.epa_gw = round_up(cvx::poly_words(L.epa_svc, L.epa_sfc), 4) + kEpaRequest + cvx::kManifoldWords;
-    for (int ng = 4; ng >= 2; ng /= 2) {
-      const int region = L.gpose > ng * L.epa_gw ? L.gpose : ng * L.epa_gw, meshw = round_up(region + GP_WORDS * m.ngeom, 4);
-      if (meshw + 4 * m.nmeshvert <= L.win) { L.epa_ng = ng; L.gpose = region; L.meshw = meshw; break; }
-    }
+    for (int ng = 4; ng >= 2 && !L.epa_ng; --ng)
+      if (region(ng * L.epa_gw)) L.epa_ng = ng;
   }
-  // contact staging (collide()): a pair table of kStagePair words per lane and kStageContact words
-  // per contact of a candidate batch, over the EPA region, which is dead once the batch's EPA ends
-  L.stage = -1;
-  if (m.njmax > 0 && L.epa == 0 && kStagePair * kLanes + kStageContact * m.nconmax <= L.gpose) L.stage = 0;
 #endif
   // Newton Hessian island blocks (packed lower triangles) and the sweep's pivot column, in FP64:
   // the blocks couple stiff contact rows with the small inertias of light objects
