@@ -75,11 +75,14 @@ constexpr int kStagePair = 18, kStageContact = 8;
 // With the scalar slots after it a world takes exactly 10 KB, so sixteen worlds fill the CU's
 // 160 KB.
 constexpr int kWindowWords = 2512;
-constexpr int kLdsScalars = 48;
-// workspace route: per-geom collision record in the LDS window during the collision stage (pose,
-// size, type, margin, gap, bounding radius, hull vertices: image word offset and count)
-enum : int { GP_POS = 0, GP_MAT = 3, GP_SIZE = 12, GP_TYPE = 15, GP_MARGIN = 16, GP_GAP = 17, GP_RBOUND = 18,
-             GP_VERT = 19, GP_NVERT = 20, GP_WORDS = 21 };     // workspace route: the misc and sv slots, in LDS after the window
+constexpr int kLdsScalars = 48;     // workspace route: the misc and sv slots, in LDS after the window
+// workspace route: per geom in the LDS window during the collision stage, first four words for the
+// broadphase (position and reach: bounding radius + margin + gap, negative for a plane, NaN on a
+// parked body; one 16-byte read), then for all geoms a record of the rest (rotation, size, type with
+// the hull's vertex count above its eight bits, margin, gap, bounding radius, hull vertices' image
+// word offset; an odd stride, so lanes reading consecutive records meet no bank twice)
+enum : int { GP_MAT = 0, GP_SIZE = 9, GP_TYPE = 12, GP_MARGIN = 13, GP_GAP = 14, GP_RBOUND = 15, GP_VERT = 16,
+             GP_RECORD = 17, GP_BROAD = 4, GP_WORDS = GP_RECORD + GP_BROAD };
 // Island sweep: block entries whose (island, row, column) a lane keeps in registers, and the words
 // per lane of the workspace route's per-substep cache of those decodes (3 per entry + 4).  The
 // workspace route is built twice, with 8 (MX_OWN default) and with 4 entries per lane: the launch
@@ -314,16 +317,19 @@ struct Ctx {
   __device__ lfloat* fi() const { return (lfloat*)params().d.workspace + L().img; }   // shared by all worlds
   __device__ double* od() const { return (double*)hwin(); }
   // geom g during collision: its record in the LDS window
-  __device__ const sfloat* grec(int g) const { return (const sfloat*)mx_lds + L().gpose + GP_WORDS * g; }
-  __device__ const sfloat* gpos(int g) const { return grec(g) + GP_POS; }
+  __device__ const sfloat* gbroad(int g) const { return (const sfloat*)mx_lds + L().gpose + GP_BROAD * g; }
+  __device__ const sfloat* grec(int g) const {
+    return (const sfloat*)mx_lds + L().gpose + GP_BROAD * m().ngeom + GP_RECORD * g;
+  }
+  __device__ const sfloat* gpos(int g) const { return gbroad(g); }
   __device__ const sfloat* gmat(int g) const { return grec(g) + GP_MAT; }
   __device__ const sfloat* gsize(int g) const { return grec(g) + GP_SIZE; }
-  __device__ int gtype(int g) const { return ((const sint*)grec(g))[GP_TYPE]; }
+  __device__ int gtype(int g) const { return ((const sint*)grec(g))[GP_TYPE] & 255; }
   __device__ float gmargin(int g) const { return grec(g)[GP_MARGIN]; }
   __device__ float ggap(int g) const { return grec(g)[GP_GAP]; }
   __device__ float grbound(int g) const { return grec(g)[GP_RBOUND]; }
   __device__ const sfloat* gvert(int g) const { return (const sfloat*)mx_lds + L().meshw + ((const sint*)grec(g))[GP_VERT]; }
-  __device__ int gnvert(int g) const { return ((const sint*)grec(g))[GP_NVERT]; }
+  __device__ int gnvert(int g) const { return ((const sint*)grec(g))[GP_TYPE] >> 8; }
 #else
   __device__ unsigned char* base() const { return mx_lds; }
   __device__ sdouble* hwin() const { return nullptr; }
@@ -2207,6 +2213,65 @@ __device__ __noinline__ bool convex_epa_rows(const Ctx& c, ConvexLane& __restric
 #endif
 }
 
+#ifdef MX_SLAB
+// The broadphase's filter of the whole pair table: the kept pairs, in table order, to the candidate
+// list; returns their count.  Its cost is the table's length: kPairBatch rounds of 64 pairs have
+// their table loads and then their geoms' 16-byte reads in flight together, and a round without
+// candidates ends with its ballot.  (One round at a time, on six to thirteen 4-byte reads in
+// branches, the LIBERO bowl-and-plate scene's 13843 pairs took 98 us of a 757 us substep.)  Out of
+// line: inlined, its registers pushed the kernel body's values to scratch.  The bound is rounded up
+// past the sums' rounding, so no pair is lost that the narrowphase's own thresholds would accept.
+constexpr int kPairBatch = 4;
+
+__device__ __noinline__ int broadphase(const Ctx& c) {
+  KModel& m = c.m();
+  int* cand = c.N(c.L().cand);
+  const int* pairs = c.IN(c.I().pair);
+  int ncand = 0;
+  for (int base = 0; base < m.npair; base += kPairBatch * kLanes) {
+    const int lane = c.lane();
+    int g1[kPairBatch], g2[kPairBatch];
+    bool keep[kPairBatch];
+    v4f a[kPairBatch], b[kPairBatch];
+#pragma unroll
+    for (int u = 0; u < kPairBatch; ++u) {
+      const int p = base + u * kLanes + lane, q = p < m.npair ? p : 0;
+      g1[u] = pairs[2 * q];
+      g2[u] = pairs[2 * q + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kPairBatch; ++u) {
+      a[u] = *(const sfloat4*)c.gbroad(g1[u]);
+      b[u] = *(const sfloat4*)c.gbroad(g2[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kPairBatch; ++u) {
+      const real dx = b[u].x - a[u].x, dy = b[u].y - a[u].y, dz = b[u].z - a[u].z;
+      const real bound = (a[u].w + b[u].w) * (1.f + 4e-6f);
+      const bool plane = a[u].w < 0.f;
+      keep[u] = dx * dx + dy * dy + dz * dz <= bound * bound && !plane;
+      if (__ballot(plane)) {   // plane against a geom's bounding sphere
+        const sfloat* gm1 = c.gmat(g1[u]);
+        const real thr = b[u].w + c.gmargin(g1[u]) + c.ggap(g1[u]);
+        if (plane) {
+          const real h = gm1[2] * dx + gm1[5] * dy + gm1[8] * dz;
+          keep[u] = h - thr <= 4e-6f * (r_abs(h) + r_abs(thr));
+        }
+      }
+      if (base + u * kLanes + lane >= m.npair) keep[u] = false;
+    }
+#pragma unroll
+    for (int u = 0; u < kPairBatch; ++u) {
+      const unsigned long long mask = __ballot(keep[u]);
+      if (!mask) continue;
+      if (keep[u]) cand[ncand + lanes_below(mask, lane)] = base + u * kLanes + lane;
+      ncand += __popcll(mask);
+    }
+  }
+  return ncand;
+}
+#endif
+
 // Broadphase over the static pair table (bounding spheres / plane half-space), narrowphase one
 // candidate per lane, deterministic compaction, contact material and frame
 // (gpu/cuda/collision/mjwarp_broadphase.cu:21-117, mjwarp_contact.cuh:42-120).
@@ -2217,15 +2282,17 @@ __device__ void collide(const Ctx& c) {
   const int* pairs = c.IN(c.I().pair);
 #ifdef MX_SLAB
   {   // the geoms' collision records into the LDS window for the whole stage
-    sfloat* gp = (sfloat*)mx_lds + c.L().gpose;
+    sfloat* bp = (sfloat*)mx_lds + c.L().gpose;
+    sfloat* gp = bp + GP_BROAD * m.ngeom;
     const real* gx = c.F(c.L().gxpos);
     const real* gm = c.F(c.L().gxmat);
     for (int g = c.lane(); g < m.ngeom; g += kLanes) {   // one lane per geom: its loads issue together
-      real x[GP_TYPE];
-      for (int k = 0; k < 3; ++k) x[GP_POS + k] = gx[3 * g + k];
+      real x[GP_TYPE], pos[3];
+      for (int k = 0; k < 3; ++k) pos[k] = gx[3 * g + k];
       for (int k = 0; k < 9; ++k) x[GP_MAT + k] = gm[9 * g + k];
       for (int k = 0; k < 3; ++k) x[GP_SIZE + k] = *c.gf(g, G_SIZE + k);
       const int type = c.gi(g, G_TYPE), id = c.gi(g, G_DATAID);
+      const bool parked = m.has_body_active && c.N(c.L().bact)[c.gi(g, G_BODY)] == 0;
       const real margin = *c.gf(g, G_MARGIN), gap = *c.gf(g, G_GAP), rbound = *c.gf(g, G_RBOUND);
       int vert = 0, nvert = 0;
       if (type == GT_MESH) {
@@ -2233,19 +2300,23 @@ __device__ void collide(const Ctx& c) {
         vert = 4 * rec[0];   // words into the vertex copy
         nvert = rec[1];
       }
-      sfloat* r = gp + GP_WORDS * g;
+      for (int k = 0; k < 3; ++k) bp[GP_BROAD * g + k] = pos[k];
+      bp[GP_BROAD * g + 3] = parked ? __builtin_nanf("") : (type == GT_PLANE ? -1.f : rbound + margin + gap);
+      sfloat* r = gp + GP_RECORD * g;
       for (int k = 0; k < GP_TYPE; ++k) r[k] = x[k];
-      ((sint*)r)[GP_TYPE] = type;
+      ((sint*)r)[GP_TYPE] = type | (nvert << 8);
       r[GP_MARGIN] = margin;
       r[GP_GAP] = gap;
       r[GP_RBOUND] = rbound;
       ((sint*)r)[GP_VERT] = vert;
-      ((sint*)r)[GP_NVERT] = nvert;
     }
     wave_copy((sfloat*)mx_lds + c.L().meshw, c.fi() + c.I().mesh, 4 * m.nmeshvert, c.lane());
     sync();
   }
 #endif
+#ifdef MX_SLAB
+  const int ncand = broadphase(c);
+#else
   int ncand = 0;
   for (int base = 0; base < m.npair; base += kLanes) {
     int p = base + c.lane();
@@ -2274,6 +2345,7 @@ __device__ void collide(const Ctx& c) {
     if (keep) cand[ncand + lanes_below(mask, c.lane())] = p;
     ncand += __popcll(mask);
   }
+#endif
   sync();
   int ncon = 0, ovf = 0;
   const int C = m.nconmax;
