@@ -601,7 +601,11 @@ struct WaveGroup {
   __device__ real max(real v) const { return wave_max(v); }
   __device__ unsigned long long ballot(bool p) const { return __ballot(p); }
   __device__ int read(int v, int j) const { return __builtin_amdgcn_readlane(v, j); }   // j uniform
-  __device__ void fence() const { __syncthreads(); }
+  __device__ void fence() const {   // one wave's own operations, in order (as sync() of the stages)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 };
 struct RowGroup {
   static constexpr int kSize = 16;

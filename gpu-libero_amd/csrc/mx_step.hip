@@ -46,13 +46,16 @@ struct Layout {
   int epa, epa_req, epa_vc, epa_fc;   // EPA polytope and request block (alias the rows during collision)
   int epa_ng, epa_gw, epa_svc, epa_sfc;   // workspace route: row-group EPA blocks (count, words, capacities)
   int stage;                          // workspace route: contact staging in the LDS window (-1: none)
-  int gpose;                          // workspace route: the geoms' collision records in the LDS window
+  int gpose, gpose0;                  // workspace route: the geoms' collision records in the LDS window (at least at gpose0)
   int meshw;                          // workspace route: the hull vertices' copy in the LDS window
   int hmap, cjmap;                    // workspace route: Hessian targets of M entries and Jacobian columns
   int cq, cqn;                        // workspace route: per-contact Hessian weights (doubles) and column counts
   int hown;                           // workspace route: the sweep's per-lane entry decodes (kSweepWords x 64)
   int ctrp;                           // workspace route: the contact trees the island tables were built for
   int win;                            // workspace route: words of the per-world LDS window
+  int nwin;                           // workspace route: the words of it that the Newton solve lays itself out in
+  int swin;                           // workspace route: the smooth stages' temporaries in the window (word)
+  int ewin, ewords;                   // wide kernel: the collision waves' EPA and staging blocks past the first
   int nfloat, dbase;
   int m7, minv, J, mjt, A, Ap, Ar, Lf, Lp, Lr, jbar, N, q, qd, dbias, eepos, eerot, eevel;
   int goalpos, goalrot, grip, R, desired, wrench, pd, posture, tau, action, gains, q0, work, ndouble;
@@ -93,6 +96,79 @@ enum : int { GP_MAT = 0, GP_SIZE = 9, GP_TYPE = 12, GP_MARGIN = 13, GP_GAP = 14,
 #endif
 constexpr int kOwn = MX_OWN;
 constexpr int kSweepWords = 3 * kOwn + 4;
+
+#ifdef MX_SLAB
+// The EPA region before the geoms' collision records grows, as far as the window has room, for what
+// shares it: first the contact staging of collide() (a pair table of kStagePair words per lane and
+// kStageContact words per contact of a candidate batch; the region is dead once the batch's EPA
+// ends), then row-group EPA (four, else three or two blocks of a small polytope, its request /
+// result words and a box-manifold clip block, side by side).
+inline void place_epa_region(Layout& L, const MxModel& m) {
+  L.epa_ng = 0;
+  L.stage = -1;
+  if (m.njmax == 0 || L.epa != 0) return;
+  L.gpose = L.gpose0;
+  L.meshw = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
+  auto region = [&](int words) {   // whether the region can take so many words; it does then
+    const int at = words > L.gpose ? words : L.gpose, meshw = round_up(at + GP_WORDS * m.ngeom, 4);
+    if (meshw + 4 * m.nmeshvert > L.win) return false;
+    L.gpose = at;
+    L.meshw = meshw;
+    return true;
+  };
+  if (region(kStagePair * kLanes + kStageContact * m.nconmax)) L.stage = 0;
+  L.epa_svc = kSmallPolyVerts < L.epa_vc ? kSmallPolyVerts : L.epa_vc;
+  L.epa_sfc = kSmallPolyFaces < L.epa_fc ? kSmallPolyFaces : L.epa_fc;
+  L.epa_gw = round_up(cvx::poly_words(L.epa_svc, L.epa_sfc), 4) + kEpaRequest + cvx::kManifoldWords;
+  for (int ng = 4; ng >= 2 && !L.epa_ng; --ng)
+    if (region(ng * L.epa_gw)) L.epa_ng = ng;
+}
+
+// The window of a launch that leaves LDS free: a batch below the sixteen worlds per CU that the
+// 10 KB window is sized for gives every world an equal share of its CU's LDS (occupancy is the same
+// either way, all the batch's worlds being resident at once).  What that buys is chosen so that a
+// world's results do not depend on the batch around it: row-group EPA and the contact staging, which
+// compute the same values as their fallbacks, and (waves > 1) the blocks of the wide kernel's further
+// waves; the Newton solve, whose Hessian rebuilds round differently when they run from a saved
+// assembly, keeps the layout of the small window (nwin).  (Row-group EPA instead of
+// one pair at a time: the LIBERO bowl-and-plate scene at 500 worlds 17.8 -> 15.1 ms per control step.)
+// Returns whether the layout for so many waves fits the share.
+constexpr int kLdsGranule = 1280;   // bytes: LDS is allocated in such units
+constexpr int kWideScalars = 16;    // wide kernel: words after the scalar slots (counts per wave)
+inline bool widen_window(Layout& L, const MxModel& m, int nworld, int ncu, int waves) {
+  if (m.njmax == 0 || ncu < 1) return false;
+  const int per_cu = (nworld + ncu - 1) / ncu;
+  const int share = MX_LDS_BUDGET / per_cu / kLdsGranule * kLdsGranule / 4 - kLdsScalars - kWideScalars;
+  const int records = GP_WORDS * m.ngeom + 4 + 4 * m.nmeshvert, staging = kStagePair * kLanes + kStageContact * m.nconmax;
+  for (int staged = 1; staged >= 0; --staged) {
+    Layout W = L;
+    if (W.epa == 0) {   // room for four row-group blocks (and the staging) before records and vertices
+      const int blocks = W.gpose0 > 4 * W.epa_gw ? W.gpose0 : 4 * W.epa_gw;
+      const int want = round_up((staged && staging > blocks ? staging : blocks) + records, 4);
+      if (waves == 1 && want > share && staged) continue;
+      if (want > W.win) W.win = waves > 1 || want < share ? want : (share > W.win ? share : W.win);
+      place_epa_region(W, m);
+    }
+    if (waves > 1) {
+      // after the first wave's window: the further collision waves' EPA and staging blocks, then the
+      // smooth stages' temporaries, which run beside the collision
+      const int total = 2 * (m.nM + m.nMdamp);
+      int smooth = 23 * m.nbody + 6 * m.nv;
+      for (int need : {2 * (W.otmp_end - W.otmp), 2 * m.nu + m.nv, 16 * m.nbody + 6 * m.njnt, 18 * m.nbody + 6 * m.nv,
+                       total <= W.nwin ? total : 0})
+        if (need > smooth) smooth = need;
+      W.ewords = W.epa == 0 ? W.gpose : 4;
+      W.ewin = round_up(W.win, 4);
+      W.swin = W.ewin + (waves - 2) * W.ewords;
+      W.win = round_up(W.swin + smooth, 4);
+    }
+    if (W.win > share) continue;
+    L = W;
+    return true;
+  }
+  return false;
+}
+#endif
 
 Layout make_layout(const MxModel& m) {
   Layout L{};
@@ -206,28 +282,9 @@ Layout make_layout(const MxModel& m) {
   // then the hull vertices (4 words each), read by every support-point search of the stage
   L.meshw = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
   if (m.njmax > 0 && m.nmeshvert > 0 && L.win < L.meshw + 4 * m.nmeshvert) L.win = round_up(L.meshw + 4 * m.nmeshvert, 4);
-  // The EPA region before the collision records grows, as far as the window as sized above has room,
-  // for what shares it: first the contact staging of collide() (a pair table of kStagePair words per
-  // lane and kStageContact words per contact of a candidate batch; the region is dead once the
-  // batch's EPA ends), then row-group EPA (four, else three or two blocks of a small polytope, its
-  // request / result words and a box-manifold clip block, side by side).
-  L.epa_ng = 0;
-  L.stage = -1;
-  if (m.njmax > 0 && L.epa == 0) {
-    auto region = [&](int words) {   // whether the region can take so many words; it does then
-      const int at = words > L.gpose ? words : L.gpose, meshw = round_up(at + GP_WORDS * m.ngeom, 4);
-      if (meshw + 4 * m.nmeshvert > L.win) return false;
-      L.gpose = at;
-      L.meshw = meshw;
-      return true;
-    };
-    if (region(kStagePair * kLanes + kStageContact * m.nconmax)) L.stage = 0;
-    L.epa_svc = kSmallPolyVerts < L.epa_vc ? kSmallPolyVerts : L.epa_vc;
-    L.epa_sfc = kSmallPolyFaces < L.epa_fc ? kSmallPolyFaces : L.epa_fc;
-    L.epa_gw = round_up(cvx::poly_words(L.epa_svc, L.epa_sfc), 4) + kEpaRequest + cvx::kManifoldWords;
-    for (int ng = 4; ng >= 2 && !L.epa_ng; --ng)
-      if (region(ng * L.epa_gw)) L.epa_ng = ng;
-  }
+  L.gpose0 = L.gpose;
+  place_epa_region(L, m);
+  L.nwin = L.win;
 #endif
   // Newton Hessian island blocks (packed lower triangles) and the sweep's pivot column, in FP64:
   // the blocks couple stiff contact rows with the small inertias of light objects
@@ -311,11 +368,14 @@ struct Ctx {
     return reinterpret_cast<unsigned char*>(params().d.workspace + (size_t)(w() + 1) * params().d.workspace_doubles);
   }
   __device__ sdouble* hwin() const { return (sdouble*)mx_lds; }   // the world's LDS window
+  // the smooth stages' part of it: the start, or (wide kernel) a part beside the collision's
+  __device__ sfloat* swin() const { return (sfloat*)mx_lds + L().swin; }
+  __device__ sint* wide() const { return (sint*)mx_lds + L().win + kLdsScalars; }   // wide kernel: counts per wave
   // the world's scalar slots (misc: 16 words, sv: 32 words) in LDS after the window
   __device__ int* MISC() const { return (int*)((sint*)mx_lds + L().win); }
   __device__ int* SV() const { return (int*)((sint*)mx_lds + L().win + 16); }
   __device__ lfloat* fi() const { return (lfloat*)params().d.workspace + L().img; }   // shared by all worlds
-  __device__ double* od() const { return (double*)hwin(); }
+  __device__ double* od() const { return (double*)(sdouble*)swin(); }
   // geom g during collision: its record in the LDS window
   __device__ const sfloat* gbroad(int g) const { return (const sfloat*)mx_lds + L().gpose + GP_BROAD * g; }
   __device__ const sfloat* grec(int g) const {
@@ -382,20 +442,16 @@ struct Ctx {
   __device__ real ctrlrange(int a, int k) const { return af(a, A_CTRLRANGE + k); }
 };
 
-#ifdef MX_SLAB
-__device__ __forceinline__ void sync() { __syncthreads(); }
-#else
-// The LDS route's stage code synchronizes its own wavefront: its workgroups hold one wave, or two
-// whose waves run different stages at once (control_step_kernel_smooth) and meet at that kernel's
-// own workgroup barriers only.  A wave's LDS and memory operations complete in order, so a wave
-// barrier between fences that keep the compiler from moving accesses across it orders its lanes'
+// Stage code synchronizes its own wavefront: a workgroup holds one wave, or several whose waves run
+// different stages at once (control_step_kernel_smooth, control_step_kernel_wide) and meet at those
+// kernels' own workgroup barriers only.  A wave's LDS and memory operations complete in order, so a
+// wave barrier between fences that keep the compiler from moving accesses across it orders its lanes'
 // accesses.
 __device__ __forceinline__ void sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-#endif
 
 // ---------------------------------------------------------------- position stage
 // Forward kinematics: MuJoCo mj_kinematics semantics (reference fused leaf
@@ -411,7 +467,7 @@ __device__ void kinematics(const Ctx& c) {
   // window (free at a substep's start; 16 nbody + 6 njnt words, which the layout guarantees), so
   // each jumping round reads its ancestors' frames at LDS latency instead of the working set's.
   const int nbw = m.nbody;
-  real* tp = (real*)(sfloat*)c.hwin();
+  real* tp = (real*)c.swin();
   real *tq = tp + 3 * nbw, *tp1 = tq + 4 * nbw, *tq1 = tp1 + 3 * nbw;
   int* anc = (int*)(tq1 + 4 * nbw);
   int* anc1 = anc + nbw;
@@ -567,17 +623,18 @@ __device__ void kinematics(const Ctx& c) {
 // together) and accumulate them in the original order, so the sums are those of the plain loop.
 constexpr int kBatch = 8;
 
-// dst[t] = src[t] for t < n, the wave's lanes striding by 64, kBatch loads in flight per lane
+// dst[t] = src[t] for t < n, the wave's lanes (or `step` threads) striding, kBatch loads in flight
+// per lane
 template <class D, class S>
-__device__ __forceinline__ void wave_copy(D* dst, const S* src, int n, int lane) {
+__device__ __forceinline__ void wave_copy(D* dst, const S* src, int n, int lane, int step = kLanes) {
   using T = decltype(+*src);   // the element type without its address space
-  for (int t0 = lane; t0 < n; t0 += kBatch * kLanes) {
+  for (int t0 = lane; t0 < n; t0 += kBatch * step) {
     T v[kBatch];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) v[u] = src[t0 + u * kLanes < n ? t0 + u * kLanes : t0];
+    for (int u = 0; u < kBatch; ++u) v[u] = src[t0 + u * step < n ? t0 + u * step : t0];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
-      if (t0 + u * kLanes < n) dst[t0 + u * kLanes] = v[u];
+      if (t0 + u * step < n) dst[t0 + u * step] = v[u];
   }
 }
 
@@ -651,7 +708,7 @@ __device__ void com_pos(const Ctx& c) {
   // Workspace route: the passes below and crb_mass() read the subtree coms, cinert and cdof from
   // copies in the LDS window (23 nbody + 6 nv words with crb_mass()'s crb, which the layout
   // guarantees); the working set receives them too for the later stages.
-  real* wscom = (real*)(sfloat*)c.hwin();
+  real* wscom = (real*)c.swin();
   real* wci = wscom + 3 * m.nbody;
   real* wcd = wci + 20 * m.nbody;
 #endif
@@ -769,9 +826,9 @@ __device__ void crb_mass(const Ctx& c) {
   real* M = c.F(c.L().M);
 #ifdef MX_SLAB
   // Workspace route: cinert and cdof from com_pos()'s window copies, crb in the window
-  const real* ci = (real*)(sfloat*)c.hwin() + 3 * m.nbody;
-  real* crb = (real*)(sfloat*)c.hwin() + 13 * m.nbody;
-  const real* cdof = (real*)(sfloat*)c.hwin() + 23 * m.nbody;
+  const real* ci = (real*)c.swin() + 3 * m.nbody;
+  real* crb = (real*)c.swin() + 13 * m.nbody;
+  const real* cdof = (real*)c.swin() + 23 * m.nbody;
 #else
   const real* ci = c.F(c.L().cinert);
   real* crb = c.F(c.L().crb);
@@ -890,8 +947,8 @@ __device__ void mass_inverse(const Ctx& c, const lreal* M, lreal* out, bool damp
   const int total = c.m().nM + (damp ? c.m().nMdamp : 0);
   const bool small = total <= 8 * kLanes;
 #ifdef MX_SLAB
-  if (2 * total <= c.L().win) {
-    sfloat* w = (sfloat*)c.hwin();
+  if (2 * total <= c.L().nwin) {
+    sfloat* w = c.swin();
     if (small) mass_inverse_in<8>(c, M, out, damp, h, w, w + total);
     else mass_inverse_in<16>(c, M, out, damp, h, w, w + total);
     return;
@@ -1038,7 +1095,7 @@ __device__ void velocity(const Ctx& c) {
   // subtree sums from copies in the LDS window (free between the rows and the controller; 18 nbody
   // + 6 nv words, which the layout guarantees); cvel and cdof_dot also go to the working set for
   // the post-constraint stage.
-  real* wcvel = (real*)(sfloat*)c.hwin();
+  real* wcvel = (real*)c.swin();
   real* wcdd = wcvel + 6 * m.nbody;
   real* cfb = wcdd + 6 * m.nv;
   real* cfrc = cfb + 6 * m.nbody;
@@ -1633,7 +1690,7 @@ __device__ void actuation(const Ctx& c) {
   // actuator's inputs, the dof's force terms, its row of M^-1 up to kRowHeld columns) before any
   // store.  Same operations in the same order as the general form below.
   constexpr int kRowHeld = 16;
-  sreal* xg = (sreal*)c.hwin();         // gear x force of each actuator
+  sreal* xg = (sreal*)c.swin();         // gear x force of each actuator
   sint* xd = (sint*)(xg + m.nu);        // the actuator's dof
   sreal* xs = xg + 2 * m.nu;            // qfrc_smooth
   const int lane = c.lane();
@@ -2003,11 +2060,13 @@ __device__ __noinline__ bool convex_begin(const Ctx& c, int g1, int g2, ConvexLa
 }
 
 // EPA of the leader lane's pair by the whole wave; the leader emits the contacts.
-__device__ __noinline__ void convex_epa(const Ctx& c, ConvexLane& __restrict__ s, RawOut& __restrict__ o, bool leader) {
+// eoff: the first word of the calling wave's EPA block in the LDS window (workspace route).
+__device__ __noinline__ void convex_epa(const Ctx& c, ConvexLane& __restrict__ s, RawOut& __restrict__ o, bool leader,
+                                        int eoff) {
   KModel& m = c.m();
 #ifdef MX_SLAB
-  sfloat* ebase = (sfloat*)c.hwin();
-  cvx::Poly p = cvx::poly_at(ebase + c.L().epa, c.L().epa_vc, c.L().epa_fc);
+  sfloat* ebase = (sfloat*)c.hwin() + eoff;
+  cvx::Poly p = cvx::poly_at(ebase, c.L().epa_vc, c.L().epa_fc);
   sfloat* rq = ebase + c.L().epa_req;
 #else
   cvx::Poly p = cvx::poly_at((sreal*)(c.f() + c.L().epa), c.L().epa_vc, c.L().epa_fc);
@@ -2057,7 +2116,7 @@ __device__ __noinline__ void convex_epa(const Ctx& c, ConvexLane& __restrict__ s
     e = cvx::epa_expand(p, m.opt_ccd_tolerance, m.epa_iterations, a, b, discrete, cvx::WaveGroup(c.lane()));
     if (e.face >= 0) nf = cvx::ld(p.proj + 3 * e.face);
     if (!cvx::multicontact_supported(a, b)) e.face = -1;
-    if (e.horizon_overflow && c.lane() == 0) c.SV()[SV_OVF] |= MX_OVERFLOW_EPA_HORIZON;
+    if (e.horizon_overflow && c.lane() == 0) atomicOr(&c.SV()[SV_OVF], MX_OVERFLOW_EPA_HORIZON);
   }
   if (leader && e.distance < gap) {
     cvx::Manifold mf = cvx::single_point(e, nf);
@@ -2106,12 +2165,13 @@ __device__ __forceinline__ void pair_material(const Ctx& c, int g1, int g2, int&
 // which the row overwrites with its result, then a box-manifold clip block), so the single-lane
 // parts (polytope build, box manifold) of the four pairs also run side by side.  Returns true on a
 // batch lane whose pair outgrew the small polytope; that pair is expanded again by convex_epa.
+// eoff: as convex_epa's.
 __device__ __noinline__ bool convex_epa_rows(const Ctx& c, ConvexLane& __restrict__ s, RawOut& __restrict__ o,
-                                              unsigned long long batch) {
+                                              unsigned long long batch, int eoff) {
 #ifdef MX_SLAB
   KModel& m = c.m();
   const int lane = c.lane(), gw = c.L().epa_gw, ps = gw - kEpaRequest - cvx::kManifoldWords;
-  sfloat* win = (sfloat*)c.hwin() + c.L().epa;
+  sfloat* win = (sfloat*)c.hwin() + eoff;
   const bool mine = ((batch >> lane) & 1ull) != 0ull;
   const int rank = __popcll(batch & ((1ull << lane) - 1ull));
   if (mine) {   // the request of this lane's pair into block `rank` (as convex_epa's leader)
@@ -2214,8 +2274,8 @@ __device__ __noinline__ bool convex_epa_rows(const Ctx& c, ConvexLane& __restric
 }
 
 #ifdef MX_SLAB
-// The broadphase's filter of the whole pair table: the kept pairs, in table order, to the candidate
-// list; returns their count.  Its cost is the table's length: kPairBatch rounds of 64 pairs have
+// The broadphase's filter of pairs [first, last) of the table: the kept pairs, in table order, to the
+// candidate list from its entry `first` on; returns their count.  Its cost is the table's length: kPairBatch rounds of 64 pairs have
 // their table loads and then their geoms' 16-byte reads in flight together, and a round without
 // candidates ends with its ballot.  (One round at a time, on six to thirteen 4-byte reads in
 // branches, the LIBERO bowl-and-plate scene's 13843 pairs took 98 us of a 757 us substep.)  Out of
@@ -2223,19 +2283,18 @@ __device__ __noinline__ bool convex_epa_rows(const Ctx& c, ConvexLane& __restric
 // past the sums' rounding, so no pair is lost that the narrowphase's own thresholds would accept.
 constexpr int kPairBatch = 4;
 
-__device__ __noinline__ int broadphase(const Ctx& c) {
-  KModel& m = c.m();
-  int* cand = c.N(c.L().cand);
+__device__ __noinline__ int broadphase(const Ctx& c, int first, int last) {
+  int* cand = c.N(c.L().cand) + first;
   const int* pairs = c.IN(c.I().pair);
   int ncand = 0;
-  for (int base = 0; base < m.npair; base += kPairBatch * kLanes) {
+  for (int base = first; base < last; base += kPairBatch * kLanes) {
     const int lane = c.lane();
     int g1[kPairBatch], g2[kPairBatch];
     bool keep[kPairBatch];
     v4f a[kPairBatch], b[kPairBatch];
 #pragma unroll
     for (int u = 0; u < kPairBatch; ++u) {
-      const int p = base + u * kLanes + lane, q = p < m.npair ? p : 0;
+      const int p = base + u * kLanes + lane, q = p < last ? p : first;
       g1[u] = pairs[2 * q];
       g2[u] = pairs[2 * q + 1];
     }
@@ -2258,7 +2317,7 @@ __device__ __noinline__ int broadphase(const Ctx& c) {
           keep[u] = h - thr <= 4e-6f * (r_abs(h) + r_abs(thr));
         }
       }
-      if (base + u * kLanes + lane >= m.npair) keep[u] = false;
+      if (base + u * kLanes + lane >= last) keep[u] = false;
     }
 #pragma unroll
     for (int u = 0; u < kPairBatch; ++u) {
@@ -2272,6 +2331,185 @@ __device__ __noinline__ int broadphase(const Ctx& c) {
 }
 #endif
 
+#ifdef MX_SLAB
+// The geoms' collision records and the hull vertices into the LDS window for the whole stage, by
+// threads tid, tid + n, ... of the world.
+__device__ __forceinline__ void collision_records(const Ctx& c, int tid, int n) {
+  KModel& m = c.m();
+  sfloat* bp = (sfloat*)mx_lds + c.L().gpose;
+  sfloat* gp = bp + GP_BROAD * m.ngeom;
+  const real* gx = c.F(c.L().gxpos);
+  const real* gm = c.F(c.L().gxmat);
+  for (int g = tid; g < m.ngeom; g += n) {   // one thread per geom: its loads issue together
+    real x[GP_TYPE], pos[3];
+    for (int k = 0; k < 3; ++k) pos[k] = gx[3 * g + k];
+    for (int k = 0; k < 9; ++k) x[GP_MAT + k] = gm[9 * g + k];
+    for (int k = 0; k < 3; ++k) x[GP_SIZE + k] = *c.gf(g, G_SIZE + k);
+    const int type = c.gi(g, G_TYPE), id = c.gi(g, G_DATAID);
+    const bool parked = m.has_body_active && c.N(c.L().bact)[c.gi(g, G_BODY)] == 0;
+    const real margin = *c.gf(g, G_MARGIN), gap = *c.gf(g, G_GAP), rbound = *c.gf(g, G_RBOUND);
+    int vert = 0, nvert = 0;
+    if (type == GT_MESH) {
+      const int* rec = c.IN(c.I().meshrec + 2 * id);
+      vert = 4 * rec[0];   // words into the vertex copy
+      nvert = rec[1];
+    }
+    for (int k = 0; k < 3; ++k) bp[GP_BROAD * g + k] = pos[k];
+    bp[GP_BROAD * g + 3] = parked ? __builtin_nanf("") : (type == GT_PLANE ? -1.f : rbound + margin + gap);
+    sfloat* r = gp + GP_RECORD * g;
+    for (int k = 0; k < GP_TYPE; ++k) r[k] = x[k];
+    ((sint*)r)[GP_TYPE] = type | (nvert << 8);
+    r[GP_MARGIN] = margin;
+    r[GP_GAP] = gap;
+    r[GP_RBOUND] = rbound;
+    ((sint*)r)[GP_VERT] = vert;
+  }
+  wave_copy((sfloat*)mx_lds + c.L().meshw, c.fi() + c.I().mesh, 4 * m.nmeshvert, tid, n);
+}
+#endif
+
+// The narrowphase of one candidate per lane (pair p of the table; -1: none): the pair's routine, then
+// EPA of the lanes whose convex pair needs it.  eoff: the calling wave's EPA block (convex_epa).
+__device__ __forceinline__ void narrow_candidates(const Ctx& c, int p, int eoff, RawOut& o, int& g1, int& g2) {
+  KModel& m = c.m();
+  const int* pairs = c.IN(c.I().pair);
+  o.n = 0;
+  o.tangent_mask = 0u;
+  g1 = g2 = 0;
+  bool pending = false;
+  ConvexLane cl;
+  if (p >= 0) {
+    g1 = pairs[2 * p];
+    g2 = pairs[2 * p + 1];
+    if (convex_pair(m, c.gtype(g1), c.gtype(g2))) {
+      if (m.convex_mpr) lane_mpr(c, g1, g2, o);
+      else pending = convex_begin(c, g1, g2, cl, o);
+    } else {
+      lane_narrowphase(c, g1, g2, pair_margin(c, g1, g2).thr, o);
+    }
+  }
+  // pairs that need EPA: up to four at a time, each expanded by a 16-lane row of the wave on a
+  // small polytope (workspace route, when the window holds them); a pair alone, and any pair
+  // that outgrew its small polytope, expanded by the whole wave on the full-size one
+  unsigned long long pend = __ballot(pending);
+#ifdef MX_SLAB
+  if (c.L().epa_ng > 1) {
+    unsigned long long again = 0ull;
+    while (__popcll(pend) > 1) {
+      unsigned long long batch = 0ull, rest = pend;
+      for (int k = 0; k < c.L().epa_ng && rest; ++k) {
+        batch |= rest & (~rest + 1ull);
+        rest &= rest - 1ull;
+      }
+      again |= __ballot(convex_epa_rows(c, cl, o, batch, eoff));
+      pend = rest;
+    }
+    pend |= again;
+  }
+#endif
+  for (; pend; pend &= pend - 1) {
+    int leader = __ffsll((long long)pend) - 1;
+    convex_epa(c, cl, o, c.lane() == leader, eoff);
+  }
+}
+
+// The lanes' contacts into the world's contact arrays from slot `ncon` on, lane l's from its `off`
+// (`total` over the wave); returns whether some found no slot.  stage: the calling wave's staging
+// block in the LDS window (workspace route; -1: each pair's lane writes its contacts itself).
+__device__ __forceinline__ bool emit_contacts(const Ctx& c, const RawOut& o, int g1, int g2, int off, int total, int ncon,
+                                              int stage) {
+  KModel& m = c.m();
+  const int C = m.nconmax;
+  int ovf = 0;
+#ifdef MX_SLAB
+  if (stage >= 0) {
+    // the pairs' records and their contacts into the LDS staging (each pair lane), then one lane
+    // per contact writes the contact's fields: stores of consecutive slots from consecutive lanes
+    sfloat* P = (sfloat*)mx_lds + stage;
+    sfloat* S = P + kStagePair * kLanes;
+    if (o.n) {
+      int dim;
+      real fr[3], solref[2], solimp[5];
+      pair_material(c, g1, g2, dim, fr, solref, solimp);
+      const PairMargin pm = pair_margin(c, g1, g2);
+      sfloat* pe = P + kStagePair * c.lane();
+      for (int k = 0; k < 3; ++k) pe[k] = fr[k];
+      pe[3] = solref[0]; pe[4] = solref[1];
+      for (int k = 0; k < 5; ++k) pe[5 + k] = solimp[k];
+      pe[10] = pm.margin - pm.gap;
+      ((sint*)pe)[11] = g1; ((sint*)pe)[12] = g2; ((sint*)pe)[13] = dim;
+      for (int k = 0; k < 3; ++k) pe[14 + k] = o.tangent[k];
+      ((sint*)pe)[17] = (int)o.tangent_mask;
+      for (int k = 0; k < o.n; ++k) {
+        const int st = off + k;
+        if (ncon + st >= C) { ovf = 1; continue; }
+        sfloat* se = S + kStageContact * st;
+        for (int j = 0; j < 3; ++j) { se[j] = o.pos[k][j]; se[3 + j] = o.normal[k][j]; }
+        se[6] = o.dist[k];
+        ((sint*)se)[7] = c.lane() | (k << 8);
+      }
+    }
+    sync();
+    const int nnew = min(total, C - ncon);
+    for (int st = c.lane(); st < nnew; st += kLanes) {
+      const sfloat* se = S + kStageContact * st;
+      const int owner = ((const sint*)se)[7], k = owner >> 8, slot = ncon + st;
+      const sfloat* pe = P + kStagePair * (owner & 255);
+      real nrm[3] = {se[3], se[4], se[5]}, fr9[9];
+      if ((((const sint*)pe)[17] >> k) & 1) {
+        real tg[3] = {pe[14], pe[15], pe[16]};
+        for (int j = 0; j < 3; ++j) { fr9[j] = nrm[j]; fr9[3 + j] = tg[j]; }
+        cross3(nrm, tg, fr9 + 6);
+      } else {
+        make_frame(nrm, fr9);
+      }
+      for (int j = 0; j < 3; ++j) c.F(c.L().cpos)[3 * slot + j] = se[j];
+      for (int j = 0; j < 9; ++j) c.F(c.L().cframe)[9 * slot + j] = fr9[j];
+      c.F(c.L().cdist)[slot] = se[6];
+      real* f5 = c.F(c.L().cfric) + 5 * slot;
+      f5[0] = pe[0]; f5[1] = pe[0]; f5[2] = pe[1]; f5[3] = pe[2]; f5[4] = pe[2];
+      for (int j = 0; j < 2; ++j) c.F(c.L().csolref)[2 * slot + j] = pe[3 + j];
+      for (int j = 0; j < 5; ++j) c.F(c.L().csolimp)[5 * slot + j] = pe[5 + j];
+      c.F(c.L().cmargin)[slot] = pe[10];
+      c.N(c.L().cgeom)[2 * slot] = ((const sint*)pe)[11];
+      c.N(c.L().cgeom)[2 * slot + 1] = ((const sint*)pe)[12];
+      c.N(c.L().cdim)[slot] = ((const sint*)pe)[13];
+    }
+    sync();
+  } else
+#endif
+  {
+    if (o.n) {
+      int dim;
+      real fr[3], solref[2], solimp[5];
+      pair_material(c, g1, g2, dim, fr, solref, solimp);
+      const PairMargin pm = pair_margin(c, g1, g2);
+      for (int k = 0; k < o.n; ++k) {
+        int slot = ncon + off + k;
+        if (slot >= C) { ovf = 1; continue; }
+        for (int j = 0; j < 3; ++j) c.F(c.L().cpos)[3 * slot + j] = o.pos[k][j];
+        real* fr9 = c.F(c.L().cframe) + 9 * slot;
+        if (o.tangent_mask & (1u << k)) {
+          for (int j = 0; j < 3; ++j) { fr9[j] = o.normal[k][j]; fr9[3 + j] = o.tangent[j]; }
+          cross3(o.normal[k], o.tangent, fr9 + 6);
+        } else {
+          make_frame(o.normal[k], fr9);
+        }
+        c.F(c.L().cdist)[slot] = o.dist[k];
+        real* f5 = c.F(c.L().cfric) + 5 * slot;
+        f5[0] = fr[0]; f5[1] = fr[0]; f5[2] = fr[1]; f5[3] = fr[2]; f5[4] = fr[2];
+        for (int j = 0; j < 2; ++j) c.F(c.L().csolref)[2 * slot + j] = solref[j];
+        for (int j = 0; j < 5; ++j) c.F(c.L().csolimp)[5 * slot + j] = solimp[j];
+        c.F(c.L().cmargin)[slot] = pm.margin - pm.gap;
+        c.N(c.L().cgeom)[2 * slot] = g1;
+        c.N(c.L().cgeom)[2 * slot + 1] = g2;
+        c.N(c.L().cdim)[slot] = dim;
+      }
+    }
+  }
+  return ovf;
+}
+
 // Broadphase over the static pair table (bounding spheres / plane half-space), narrowphase one
 // candidate per lane, deterministic compaction, contact material and frame
 // (gpu/cuda/collision/mjwarp_broadphase.cu:21-117, mjwarp_contact.cuh:42-120).
@@ -2281,41 +2519,11 @@ __device__ void collide(const Ctx& c) {
   int* cand = c.N(c.L().cand);
   const int* pairs = c.IN(c.I().pair);
 #ifdef MX_SLAB
-  {   // the geoms' collision records into the LDS window for the whole stage
-    sfloat* bp = (sfloat*)mx_lds + c.L().gpose;
-    sfloat* gp = bp + GP_BROAD * m.ngeom;
-    const real* gx = c.F(c.L().gxpos);
-    const real* gm = c.F(c.L().gxmat);
-    for (int g = c.lane(); g < m.ngeom; g += kLanes) {   // one lane per geom: its loads issue together
-      real x[GP_TYPE], pos[3];
-      for (int k = 0; k < 3; ++k) pos[k] = gx[3 * g + k];
-      for (int k = 0; k < 9; ++k) x[GP_MAT + k] = gm[9 * g + k];
-      for (int k = 0; k < 3; ++k) x[GP_SIZE + k] = *c.gf(g, G_SIZE + k);
-      const int type = c.gi(g, G_TYPE), id = c.gi(g, G_DATAID);
-      const bool parked = m.has_body_active && c.N(c.L().bact)[c.gi(g, G_BODY)] == 0;
-      const real margin = *c.gf(g, G_MARGIN), gap = *c.gf(g, G_GAP), rbound = *c.gf(g, G_RBOUND);
-      int vert = 0, nvert = 0;
-      if (type == GT_MESH) {
-        const int* rec = c.IN(c.I().meshrec + 2 * id);
-        vert = 4 * rec[0];   // words into the vertex copy
-        nvert = rec[1];
-      }
-      for (int k = 0; k < 3; ++k) bp[GP_BROAD * g + k] = pos[k];
-      bp[GP_BROAD * g + 3] = parked ? __builtin_nanf("") : (type == GT_PLANE ? -1.f : rbound + margin + gap);
-      sfloat* r = gp + GP_RECORD * g;
-      for (int k = 0; k < GP_TYPE; ++k) r[k] = x[k];
-      ((sint*)r)[GP_TYPE] = type | (nvert << 8);
-      r[GP_MARGIN] = margin;
-      r[GP_GAP] = gap;
-      r[GP_RBOUND] = rbound;
-      ((sint*)r)[GP_VERT] = vert;
-    }
-    wave_copy((sfloat*)mx_lds + c.L().meshw, c.fi() + c.I().mesh, 4 * m.nmeshvert, c.lane());
-    sync();
-  }
+  collision_records(c, c.lane(), kLanes);
+  sync();
 #endif
 #ifdef MX_SLAB
-  const int ncand = broadphase(c);
+  const int ncand = broadphase(c, 0, m.npair);
 #else
   int ncand = 0;
   for (int base = 0; base < m.npair; base += kLanes) {
@@ -2347,139 +2555,15 @@ __device__ void collide(const Ctx& c) {
   }
 #endif
   sync();
-  int ncon = 0, ovf = 0;
-  const int C = m.nconmax;
+  int ncon = 0;
+  bool ovf = false;
   for (int base = 0; base < ncand; base += kLanes) {
-    int q = base + c.lane();
     RawOut o;
-    o.n = 0;
-    o.tangent_mask = 0u;
-    int g1 = 0, g2 = 0;
-    bool pending = false;
-    ConvexLane cl;
-    if (q < ncand) {
-      int p = cand[q];
-      g1 = pairs[2 * p];
-      g2 = pairs[2 * p + 1];
-      if (convex_pair(m, c.gtype(g1), c.gtype(g2))) {
-        if (m.convex_mpr) lane_mpr(c, g1, g2, o);
-        else pending = convex_begin(c, g1, g2, cl, o);
-      } else {
-        lane_narrowphase(c, g1, g2, pair_margin(c, g1, g2).thr, o);
-      }
-    }
-    // pairs that need EPA: up to four at a time, each expanded by a 16-lane row of the wave on a
-    // small polytope (workspace route, when the window holds them); a pair alone, and any pair
-    // that outgrew its small polytope, expanded by the whole wave on the full-size one
-    unsigned long long pend = __ballot(pending);
-#ifdef MX_SLAB
-    if (c.L().epa_ng > 1) {
-      unsigned long long again = 0ull;
-      while (__popcll(pend) > 1) {
-        unsigned long long batch = 0ull, rest = pend;
-        for (int k = 0; k < c.L().epa_ng && rest; ++k) {
-          batch |= rest & (~rest + 1ull);
-          rest &= rest - 1ull;
-        }
-        again |= __ballot(convex_epa_rows(c, cl, o, batch));
-        pend = rest;
-      }
-      pend |= again;
-    }
-#endif
-    for (; pend; pend &= pend - 1) {
-      int leader = __ffsll((long long)pend) - 1;
-      convex_epa(c, cl, o, c.lane() == leader);
-    }
-    int total;
-    int off = wave_excl_scan(o.n, c.lane(), total);
-#ifdef MX_SLAB
-    if (c.L().stage >= 0) {
-      // the pairs' records and their contacts into the LDS staging (each pair lane), then one lane
-      // per contact writes the contact's fields: stores of consecutive slots from consecutive lanes
-      sfloat* P = (sfloat*)mx_lds + c.L().stage;
-      sfloat* S = P + kStagePair * kLanes;
-      if (o.n) {
-        int dim;
-        real fr[3], solref[2], solimp[5];
-        pair_material(c, g1, g2, dim, fr, solref, solimp);
-        const PairMargin pm = pair_margin(c, g1, g2);
-        sfloat* pe = P + kStagePair * c.lane();
-        for (int k = 0; k < 3; ++k) pe[k] = fr[k];
-        pe[3] = solref[0]; pe[4] = solref[1];
-        for (int k = 0; k < 5; ++k) pe[5 + k] = solimp[k];
-        pe[10] = pm.margin - pm.gap;
-        ((sint*)pe)[11] = g1; ((sint*)pe)[12] = g2; ((sint*)pe)[13] = dim;
-        for (int k = 0; k < 3; ++k) pe[14 + k] = o.tangent[k];
-        ((sint*)pe)[17] = (int)o.tangent_mask;
-        for (int k = 0; k < o.n; ++k) {
-          const int st = off + k;
-          if (ncon + st >= C) { ovf = 1; continue; }
-          sfloat* se = S + kStageContact * st;
-          for (int j = 0; j < 3; ++j) { se[j] = o.pos[k][j]; se[3 + j] = o.normal[k][j]; }
-          se[6] = o.dist[k];
-          ((sint*)se)[7] = c.lane() | (k << 8);
-        }
-      }
-      sync();
-      const int nnew = min(total, C - ncon);
-      for (int st = c.lane(); st < nnew; st += kLanes) {
-        const sfloat* se = S + kStageContact * st;
-        const int owner = ((const sint*)se)[7], k = owner >> 8, slot = ncon + st;
-        const sfloat* pe = P + kStagePair * (owner & 255);
-        real nrm[3] = {se[3], se[4], se[5]}, fr9[9];
-        if ((((const sint*)pe)[17] >> k) & 1) {
-          real tg[3] = {pe[14], pe[15], pe[16]};
-          for (int j = 0; j < 3; ++j) { fr9[j] = nrm[j]; fr9[3 + j] = tg[j]; }
-          cross3(nrm, tg, fr9 + 6);
-        } else {
-          make_frame(nrm, fr9);
-        }
-        for (int j = 0; j < 3; ++j) c.F(c.L().cpos)[3 * slot + j] = se[j];
-        for (int j = 0; j < 9; ++j) c.F(c.L().cframe)[9 * slot + j] = fr9[j];
-        c.F(c.L().cdist)[slot] = se[6];
-        real* f5 = c.F(c.L().cfric) + 5 * slot;
-        f5[0] = pe[0]; f5[1] = pe[0]; f5[2] = pe[1]; f5[3] = pe[2]; f5[4] = pe[2];
-        for (int j = 0; j < 2; ++j) c.F(c.L().csolref)[2 * slot + j] = pe[3 + j];
-        for (int j = 0; j < 5; ++j) c.F(c.L().csolimp)[5 * slot + j] = pe[5 + j];
-        c.F(c.L().cmargin)[slot] = pe[10];
-        c.N(c.L().cgeom)[2 * slot] = ((const sint*)pe)[11];
-        c.N(c.L().cgeom)[2 * slot + 1] = ((const sint*)pe)[12];
-        c.N(c.L().cdim)[slot] = ((const sint*)pe)[13];
-      }
-      sync();
-    } else
-#endif
-    {
-      if (o.n) {
-        int dim;
-        real fr[3], solref[2], solimp[5];
-        pair_material(c, g1, g2, dim, fr, solref, solimp);
-        const PairMargin pm = pair_margin(c, g1, g2);
-        for (int k = 0; k < o.n; ++k) {
-          int slot = ncon + off + k;
-          if (slot >= C) { ovf = 1; continue; }
-          for (int j = 0; j < 3; ++j) c.F(c.L().cpos)[3 * slot + j] = o.pos[k][j];
-          real* fr9 = c.F(c.L().cframe) + 9 * slot;
-          if (o.tangent_mask & (1u << k)) {
-            for (int j = 0; j < 3; ++j) { fr9[j] = o.normal[k][j]; fr9[3 + j] = o.tangent[j]; }
-            cross3(o.normal[k], o.tangent, fr9 + 6);
-          } else {
-            make_frame(o.normal[k], fr9);
-          }
-          c.F(c.L().cdist)[slot] = o.dist[k];
-          real* f5 = c.F(c.L().cfric) + 5 * slot;
-          f5[0] = fr[0]; f5[1] = fr[0]; f5[2] = fr[1]; f5[3] = fr[2]; f5[4] = fr[2];
-          for (int j = 0; j < 2; ++j) c.F(c.L().csolref)[2 * slot + j] = solref[j];
-          for (int j = 0; j < 5; ++j) c.F(c.L().csolimp)[5 * slot + j] = solimp[j];
-          c.F(c.L().cmargin)[slot] = pm.margin - pm.gap;
-          c.N(c.L().cgeom)[2 * slot] = g1;
-          c.N(c.L().cgeom)[2 * slot + 1] = g2;
-          c.N(c.L().cdim)[slot] = dim;
-        }
-      }
-    }
-    ncon = min(ncon + total, C);
+    int g1, g2, total;
+    narrow_candidates(c, base + c.lane() < ncand ? cand[base + c.lane()] : -1, c.L().epa, o, g1, g2);
+    const int off = wave_excl_scan(o.n, c.lane(), total);
+    ovf |= emit_contacts(c, o, g1, g2, off, total, ncon, c.L().stage);
+    ncon = min(ncon + total, m.nconmax);
   }
   ovf = __any(ovf);
   if (c.lane() == 0) {
@@ -4028,7 +4112,7 @@ __device__ void newton_solve(const Ctx& c, const V& v) {
 // (unused while the blocks and weights live in the window).
 template <class V>
 __device__ __forceinline__ void saved_assembly(const Ctx& c, V& v, sfloat* wf, int used, int htotal, int ncon) {
-  if (used + 2 * htotal + 18 * ncon <= c.L().win) {
+  if (used + 2 * htotal + 18 * ncon <= c.L().nwin) {
     v.Hs = (double*)(sdouble*)(wf + used);
     v.dq = v.Hs + htotal;
   } else {
@@ -4072,7 +4156,7 @@ __device__ void newton(const Ctx& c) {
     // the rows and contacts: five floats per row, eight per contact, then two 16-bit values per
     // row and three per contact
     const int rows = 6 * nefc + 8 * ncon + ((3 * ncon + 1) >> 1);
-    if (base <= c.L().win) {
+    if (base <= c.L().nwin) {
       sfloat* wf = (sfloat*)c.hwin();
       sfloat* jval = wf + hwords;
       sint* jmap = (sint*)(wf + hwords + 3 * jw);
@@ -4083,7 +4167,7 @@ __device__ void newton(const Ctx& c) {
       const real* gv = c.F(c.L().cjval);
       const int* gi = c.N(c.L().cjidx);
       wave_copy2(jval, gv, 3 * jw, jidx, gi, jw, c.lane());
-      if (base + rows <= c.L().win) {
+      if (base + rows <= c.L().nwin) {
         // the rows and contacts too: every row and contact access of the solve stays in LDS
         WinView wv{jval, jidx, jmap, qcon, c.hwin(), c.hwin() + htotal, hq, qn, xs};
         sfloat* rf = wf + base;
@@ -4132,7 +4216,7 @@ __device__ void newton(const Ctx& c) {
       newton_solve(c, wv);
       return;
     }
-    if (hwords <= c.L().win) {   // the island blocks and the contact weights alone
+    if (hwords <= c.L().nwin) {   // the island blocks and the contact weights alone
       HWinView hv{c.f() + c.L().cjval, c.n() + c.L().cjidx, jmap, c.f() + c.L().qcon, c.hwin(), c.hwin() + htotal, hq,
                   c.n() + c.L().cqn, nullptr};
       working_set_rows(c, hv);
@@ -4470,6 +4554,28 @@ constexpr int kPaceGroups = 8, kPaceStride = 64;
 __device__ __align__(256) unsigned int g_substeps_started[kPaceGroups * kPaceStride];
 #endif
 
+// MX_FLAG_BOOTSTRAP: the goal becomes the end-effector pose.
+__device__ __forceinline__ void bootstrap_goal(const Ctx& c) {
+  KModel& m = c.m();
+  const real* sp = c.F(c.L().sxpos) + 3 * m.osc_site;
+  const real* sr = c.F(c.L().sxmat) + 9 * m.osc_site;
+  if (c.lane() < 3) c.D(c.L().goalpos)[c.lane()] = sp[c.lane()];
+  if (c.lane() < 9) c.D(c.L().goalrot)[c.lane()] = sr[c.lane()];
+  if (c.lane() < 2) c.D(c.L().grip)[c.lane()] = 0.0;
+  if (c.lane() == 0) c.MISC()[kCtrlErr] = 0;
+  sync();
+}
+
+// The substep's rows, contacts and Newton iterations, summed over the launch.
+__device__ __forceinline__ void add_stats(const Ctx& c) {
+  if (c.lane() != 0) return;
+  int* sv = c.SV();
+  sv[SV_STAT] += sv[SV_NEFC];
+  sv[SV_STAT + 1] += sv[SV_NCON];
+  sv[SV_STAT + 2] += sv[SV_NITER];
+  sv[SV_STAT + 3] += sv[SV_NITER] * sv[SV_NEFC];
+}
+
 template <bool kRows>
 // The parameter block is read through params() (the kernel argument segment), never through the
 // by-value parameter, so no private copy of it is made.
@@ -4532,26 +4638,12 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
       make_rows(c);
     }
     velocity(c);
-    if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) {
-      const real* sp = c.F(L.sxpos) + 3 * m.osc_site;
-      const real* sr = c.F(L.sxmat) + 9 * m.osc_site;
-      if (c.lane() < 3) c.D(L.goalpos)[c.lane()] = sp[c.lane()];
-      if (c.lane() < 9) c.D(L.goalrot)[c.lane()] = sr[c.lane()];
-      if (c.lane() < 2) c.D(L.grip)[c.lane()] = 0.0;
-      if (c.lane() == 0) c.MISC()[kCtrlErr] = 0;
-      sync();
-    }
+    if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) bootstrap_goal(c);
     if (!(flags & MX_FLAG_NO_CONTROL)) control<false>(c, policy, s == substeps - 1 || (flags & MX_FLAG_NO_INTEGRATE));
     actuation(c);
     if (kRows) {
       newton(c);
-      if (c.lane() == 0) {   // the substep's rows, contacts and Newton iterations, summed over the launch
-        int* sv = c.SV();
-        sv[SV_STAT] += sv[SV_NEFC];
-        sv[SV_STAT + 1] += sv[SV_NCON];
-        sv[SV_STAT + 2] += sv[SV_NITER];
-        sv[SV_STAT + 3] += sv[SV_NITER] * sv[SV_NEFC];
-      }
+      add_stats(c);
     } else {
       for (int i = c.lane(); i < m.nv; i += kLanes) {
         c.F(L.qacc)[i] = c.F(L.qacc_smooth)[i];
@@ -4577,6 +4669,136 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   publish_derived(c);
   store_world(c, integrated);
 }
+
+#ifdef MX_SLAB
+// The same control step with kWaves wavefronts per world, for batches that leave wave slots free
+// (launch_kernel): there a substep is one wave's latency, and most of it is work that need not wait
+// for the rest.  All waves make the collision records and filter the pair table (a part each); then
+// waves 0 .. kWaves - 2 run the narrowphase and EPA of a share of the candidates each, while the last
+// wave runs the stages that need the positions only: com, mass matrix and inverses, velocity, the
+// FP64 controller, actuation.  The contacts are written in candidate order, so they are those of the
+// one-wave kernel; constraint rows, Newton and the rest run on wave 0.  The waves meet at this
+// kernel's workgroup barriers, which all of them reach in the same order (every loop bound and branch
+// around a barrier is uniform over the workgroup); between two barriers they write disjoint parts of
+// the working set and of the window (Layout::ewin, swin).  Results are bit for bit those of
+// control_step_kernel<true>: the same functions on the same values.
+template <int kWaves>
+__global__ __launch_bounds__(kWaves * kLanes, kMinWaves(true)) void control_step_kernel_wide(Params) {
+  {
+    typedef const __attribute__((address_space(4))) unsigned char KByte;
+    KByte* seg = (KByte*)__builtin_amdgcn_kernarg_segment_ptr();
+    if (seg + sizeof(Params) != (KByte*)__builtin_amdgcn_implicitarg_ptr()) {
+      KParams& kp = *(KParams*)seg;
+      if (threadIdx.x == 0 && (int)blockIdx.x < kp.d.nworld) kp.d.overflow[blockIdx.x] |= MX_OVERFLOW_LAUNCH;
+      return;
+    }
+  }
+  KParams& p = params();
+  KModel& m = p.m;
+  KLayout& L = p.L;
+  const int substeps = p.substeps, flags = p.flags;
+  const int w = blockIdx.x;
+  if (w >= p.d.nworld) return;
+  if (p.mask && !p.mask[w]) return;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kLanes);
+  constexpr int kSmooth = kWaves - 1;          // the wave of the smooth stages; the others collide
+  constexpr int kRound = kSmooth * kLanes;     // candidates of a narrowphase round
+  const Ctx c;
+  if (wave == 0) load_world(c);
+  bool damped = false;
+  if (!(m.opt_disableflags & (1 << 15)))
+    for (int i = 0; i < m.nv; ++i) damped |= c.df(i, D_DAMP) > 0.f;
+  // this wave's part of the pair table, in whole batches of the filter
+  const int part = (m.npair + kWaves * kPairBatch * kLanes - 1) / (kWaves * kPairBatch * kLanes) * (kPairBatch * kLanes);
+  const int eoff = wave == 0 ? L.epa : L.ewin + (wave - 1) * L.ewords;
+  const int stage = L.stage < 0 ? -1 : (wave == 0 ? L.stage : eoff);
+  sint* counts = c.wide();      // candidates of each wave's part, then (two rounds in turn) contacts of each wave
+  int integrated = 0;
+  for (int s = 0; s < substeps; ++s) {
+    const int policy = (flags & MX_FLAG_POLICY_FIRST) && s == 0;
+    const bool last = (flags & MX_FLAG_NO_INTEGRATE) || s == substeps - 1;
+    if (wave == 0) kinematics(c);
+    __syncthreads();
+    collision_records(c, (int)threadIdx.x, kWaves * kLanes);
+    __syncthreads();
+    {
+      const int first = wave * part, end = min(first + part, m.npair);
+      const int n = first < end ? broadphase(c, first, end) : 0;
+      if (c.lane() == 0) counts[wave] = n;
+    }
+    __syncthreads();
+    int before[kWaves + 1];     // candidates of the parts before each wave's
+    before[0] = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) before[k + 1] = before[k] + __builtin_amdgcn_readfirstlane(counts[k]);
+    const int ncand = before[kWaves], rounds = max(1, (ncand + kRound - 1) / kRound);
+    int ncon = 0;
+    bool ovf = false;
+    for (int r = 0; r < rounds; ++r) {
+      RawOut o;
+      int g1 = 0, g2 = 0, off = 0, total = 0;
+      sint* made = counts + kWaves + (r & 1) * kWaves;
+      if (wave != kSmooth) {
+        // the round's candidates in equal shares, in order
+        const int left = min(ncand - r * kRound, kRound), share = (left + kSmooth - 1) / kSmooth;
+        const int q = r * kRound + wave * share + c.lane();
+        int pair = -1;
+        if (c.lane() < share && q < r * kRound + left) {
+          int at = q;           // the q-th candidate: entry q - before[k] of part k
+#pragma unroll
+          for (int k = 0; k < kWaves; ++k)
+            if (q >= before[k] && q < before[k + 1]) at = k * part + q - before[k];
+          pair = c.N(L.cand)[at];
+        }
+        narrow_candidates(c, pair, eoff, o, g1, g2);
+        off = wave_excl_scan(o.n, c.lane(), total);
+        if (c.lane() == 0) made[wave] = total;
+      } else if (r == 0) {
+        com_pos(c);
+        crb_mass(c);
+        mass_inverse(c, c.R(L.M), c.R(L.Minv), damped, m.opt_timestep);
+        velocity(c);
+        if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) bootstrap_goal(c);
+        if (!(flags & MX_FLAG_NO_CONTROL)) control<false>(c, policy, last);
+        actuation(c);
+      }
+      __syncthreads();
+      int base = ncon, all = 0;
+#pragma unroll
+      for (int k = 0; k < kSmooth; ++k) {
+        const int n = __builtin_amdgcn_readfirstlane(made[k]);
+        if (k < wave) base += n;
+        all += n;
+      }
+      if (wave != kSmooth) ovf |= emit_contacts(c, o, g1, g2, off, total, min(base, m.nconmax), stage);
+      ncon = min(ncon + all, m.nconmax);
+    }
+    if (wave != kSmooth && __any(ovf) && c.lane() == 0) atomicOr(&c.SV()[SV_OVF], MX_OVERFLOW_NARROWPHASE);
+    if (wave == 0 && c.lane() == 0) c.SV()[SV_NCON] = ncon;
+    __syncthreads();
+    if (wave == 0) {
+      make_rows(c);
+      newton(c);
+      add_stats(c);
+      if (last) {
+        post_constraint<true>(c);
+        publish_constraints(c);
+        sync();
+      }
+      if (!(flags & MX_FLAG_NO_INTEGRATE)) {
+        euler(c, damped);
+        if (p.obs.nspec > 0) sample_plan(c);
+      }
+    }
+    if (flags & MX_FLAG_NO_INTEGRATE) break;
+    ++integrated;
+  }
+  if (wave == 0) {
+    publish_derived(c);
+    store_world(c, integrated);
+  }
+}
+#endif
 
 #ifndef MX_SLAB
 // The smooth path (models without constraint rows, LDS route) with two wavefronts per world, for
@@ -4627,15 +4849,7 @@ __global__ __launch_bounds__(2 * kLanes, 2) void control_step_kernel_smooth(Para
       velocity(c);
       mass_inverse(c, c.R(L.M), c.R(L.Minv), damped, m.opt_timestep);
     } else {
-      if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) {
-        const real* sp = c.F(L.sxpos) + 3 * m.osc_site;
-        const real* sr = c.F(L.sxmat) + 9 * m.osc_site;
-        if (c.lane() < 3) c.D(L.goalpos)[c.lane()] = sp[c.lane()];
-        if (c.lane() < 9) c.D(L.goalrot)[c.lane()] = sr[c.lane()];
-        if (c.lane() < 2) c.D(L.grip)[c.lane()] = 0.0;
-        if (c.lane() == 0) c.MISC()[kCtrlErr] = 0;
-        sync();
-      }
+      if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) bootstrap_goal(c);
       if (!(flags & MX_FLAG_NO_CONTROL)) control<true>(c, policy, last);
     }
     __syncthreads();
@@ -4699,19 +4913,24 @@ __global__ __launch_bounds__(256) void image_kernel(Params) {
 #endif
 
 #ifdef MX_SLAB
-// Whether a launch's worlds are all resident at once: each CU holds 4 waves per SIMD (the kernel's
-// register budget) or fewer when their LDS windows fill its 160 KB.
-static bool all_resident(int nworld, size_t shared) {
-  static int ncu[64];   // per device, filled on first use (a benign race: every writer stores the same)
+// The current device's CU count (0 when it cannot be had), asked once per device.
+static int cu_count() {
+  static int ncu[64];   // filled on first use (a benign race: every writer stores the same)
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   if (ncu[dev] <= 0) {
     int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) return false;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) return 0;
     ncu[dev] = v;
   }
-  const long long by_lds = 163840 / (long long)shared, per_cu = by_lds < 4 * kMinWaves(true) ? by_lds : 4 * kMinWaves(true);
-  return (long long)nworld <= (long long)ncu[dev] * per_cu;
+  return ncu[dev];
+}
+
+// Whether a launch's worlds are all resident at once: each CU holds 4 waves per SIMD (the kernel's
+// register budget) or fewer when their LDS windows fill its 160 KB.
+static bool all_resident(int nworld, size_t shared, int ncu) {
+  const long long by_lds = MX_LDS_BUDGET / (long long)shared, per_cu = by_lds < 4 * kMinWaves(true) ? by_lds : 4 * kMinWaves(true);
+  return (long long)nworld <= (long long)ncu * per_cu;
 }
 #endif
 
@@ -4720,9 +4939,26 @@ int launch_kernel(const MxModel* m, const MxData* d, const int32_t* mask, int su
   MxObsPlan none{};
   Params p{*m, *d, make_layout(*m), image_layout(*m), substeps, flags, mask, obs ? *obs : none, 0};
 #ifdef MX_SLAB
-  const size_t shared = (p.L.win + kLdsScalars) * sizeof(float);   // the LDS window, then misc and sv
-  p.pace = all_resident(d->nworld, shared) ? 1 : 0;
+  const int ncu = cu_count();
+  // Waves per world: as many as keep every world resident in the CU's sixteen wave slots, four at
+  // most.  Control step with one, two and four waves: C3 x67 5.17, 4.33, 4.00 ms; C1 x2 4.14, 3.34,
+  // 3.29; the LIBERO bowl-and-plate scene x500 15.1, 14.2, 11.2; C3 x1024 (four worlds per CU) 6.21,
+  // 5.38, 5.20; C3 x2048 (eight) 6.89 with one wave, 5.97 with two.  Eight waves gained 3 % on
+  // LIBERO and lost 1 to 3 % elsewhere.
+  const int per_cu = ncu > 0 ? (d->nworld + ncu - 1) / ncu : 16;
+  int waves = m->njmax == 0 || per_cu > 8 ? 1 : (per_cu > 4 ? 2 : 4);
+  while (waves > 1 && !widen_window(p.L, *m, d->nworld, ncu, waves)) waves /= 2;
+  if (waves == 1) widen_window(p.L, *m, d->nworld, ncu, 1);
+  const size_t shared = (p.L.win + kLdsScalars + (waves > 1 ? kWideScalars : 0)) * sizeof(float);   // the LDS window, then misc and sv
+  p.pace = waves == 1 && all_resident(d->nworld, shared, ncu) ? 1 : 0;
   hipLaunchKernelGGL(image_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, p);
+  if (waves > 1) {
+    if (waves == 4)
+      hipLaunchKernelGGL(control_step_kernel_wide<4>, dim3(d->nworld), dim3(4 * kLanes), shared, (hipStream_t)stream, p);
+    else
+      hipLaunchKernelGGL(control_step_kernel_wide<2>, dim3(d->nworld), dim3(2 * kLanes), shared, (hipStream_t)stream, p);
+    return (int)hipGetLastError();
+  }
 #else
   const size_t shared = p.L.bytes;
 #endif
