@@ -180,6 +180,28 @@ def pack_observations(plan, values):
     return result
 
 
+def pack_batch(plan, values):
+    """pack_observations for many worlds at once, ``values`` (n, width): name -> array stacked over
+    the worlds, the same names in the same order as one world's dict."""
+    values = np.asarray(values)
+    n = len(values)
+    if values.shape != (n, plan.width):
+        raise ValueError('observed buffer shape %s, expected (n, %d)' % (values.shape, plan.width))
+    offsets = plan.offsets
+    result, groups = OrderedDict(), OrderedDict()
+    for s in plan.specs:
+        if s.enabled and s.active:
+            data = values[:, offsets[s.name]:offsets[s.name] + s.width].copy()
+            value = data[:, 0] if s.shape == (1,) else data.reshape((n,) + tuple(s.shape))
+            result[s.name] = value
+            groups.setdefault(s.modality + '-state', []).append(value if value.ndim > 1 else value[:, None])
+    if plan.order:
+        result = OrderedDict((name, result[name]) for name in plan.order if name in result)
+    for modality, group in groups.items():
+        result[modality] = np.concatenate(group, axis=-1)
+    return result
+
+
 class DeviceObservations:
     """A plan's metadata and per-world sampling state in device tensors, bound to MxObsPlan."""
 
