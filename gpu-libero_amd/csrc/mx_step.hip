@@ -4576,6 +4576,7 @@ __device__ __forceinline__ void add_stats(const Ctx& c) {
   sv[SV_STAT + 3] += sv[SV_NITER] * sv[SV_NEFC];
 }
 
+#ifdef MX_SLAB
 template <bool kRows>
 // The parameter block is read through params() (the kernel argument segment), never through the
 // by-value parameter, so no private copy of it is made.
@@ -4605,7 +4606,6 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   if (!(m.opt_disableflags & (1 << 15)))
     for (int i = 0; i < m.nv; ++i) damped |= c.df(i, D_DAMP) > 0.f;
   int integrated = 0;
-#ifdef MX_SLAB
   // A launch lasts as long as its slowest world, and the worlds of one CU share its SIMDs: a world
   // whose substeps trail its group's mean by more than one and a half raises its wave's issue
   // priority until it catches up.  Each substep start adds one to the group's counter (a relaxed
@@ -4616,10 +4616,8 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   const unsigned int nw = (unsigned int)((p.d.nworld - (w & (kPaceGroups - 1)) + kPaceGroups - 1) / kPaceGroups);
   unsigned int* pace_ctr = g_substeps_started + (w & (kPaceGroups - 1)) * kPaceStride;
   const bool pace = kRows && p.pace;
-#endif
   for (int s = 0; s < substeps; ++s) {
     const int policy = (flags & MX_FLAG_POLICY_FIRST) && s == 0;
-#ifdef MX_SLAB
     if (pace) {
       // at this world's start of substep s - 1 the group's worlds had started before / nw
       // substeps on average, against this world's s - 1: behind by more than 1.5 substeps
@@ -4628,7 +4626,6 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
       else __builtin_amdgcn_s_setprio(0);
       if (threadIdx.x == 0) started = __hip_atomic_fetch_add(pace_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-#endif
     kinematics(c);
     com_pos(c);
     crb_mass(c);
@@ -4670,7 +4667,6 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   store_world(c, integrated);
 }
 
-#ifdef MX_SLAB
 // The same control step with kWaves wavefronts per world, for batches that leave wave slots free
 // (launch_kernel): there a substep is one wave's latency, and most of it is work that need not wait
 // for the rest.  All waves make the collision records and filter the pair table (a part each); then
@@ -4801,6 +4797,77 @@ __global__ __launch_bounds__(kWaves * kLanes, kMinWaves(true)) void control_step
 #endif
 
 #ifndef MX_SLAB
+// The LDS route's control step of models with constraint rows, with two wavefronts per world: while
+// wave 0 collides, wave 1 runs the stages that need the positions only (com, mass matrix and
+// inverses, velocity, the FP64 controller, actuation); everything else is wave 0's.  A CU holds one
+// or two such worlds in its LDS, so the second wave's slot is free.  Between the workgroup barriers
+// the waves write disjoint parts of the working set (the EPA polytope aliases the rows, which wave 1
+// does not touch).  (FP64 route, C3 x300: 12.1 -> 10.6 ms per control step.)
+__global__ __launch_bounds__(2 * kLanes, kMinWaves(true)) void control_step_kernel_rows2(Params) {
+  {
+    typedef const __attribute__((address_space(4))) unsigned char KByte;
+    KByte* seg = (KByte*)__builtin_amdgcn_kernarg_segment_ptr();
+    if (seg + sizeof(Params) != (KByte*)__builtin_amdgcn_implicitarg_ptr()) {
+      KParams& kp = *(KParams*)seg;
+      if (threadIdx.x == 0 && (int)blockIdx.x < kp.d.nworld) kp.d.overflow[blockIdx.x] |= MX_OVERFLOW_LAUNCH;
+      return;
+    }
+  }
+  KParams& p = params();
+  KModel& m = p.m;
+  KLayout& L = p.L;
+  const int substeps = p.substeps, flags = p.flags;
+  const int w = blockIdx.x;
+  if (w >= p.d.nworld) return;
+  if (p.mask && !p.mask[w]) return;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kLanes);
+  const Ctx c;
+  if (wave == 0) load_world(c);
+  __syncthreads();
+  bool damped = false;
+  if (!(m.opt_disableflags & (1 << 15)))
+    for (int i = 0; i < m.nv; ++i) damped |= c.df(i, D_DAMP) > 0.f;
+  int integrated = 0;
+  for (int s = 0; s < substeps; ++s) {
+    const int policy = (flags & MX_FLAG_POLICY_FIRST) && s == 0;
+    const bool last = (flags & MX_FLAG_NO_INTEGRATE) || s == substeps - 1;
+    if (wave == 0) kinematics(c);
+    __syncthreads();
+    if (wave == 0) {
+      collide(c);
+    } else {
+      com_pos(c);
+      crb_mass(c);
+      mass_inverse(c, c.R(L.M), c.R(L.Minv), damped, m.opt_timestep);
+      velocity(c);
+      if ((flags & MX_FLAG_BOOTSTRAP) && s == 0) bootstrap_goal(c);
+      if (!(flags & MX_FLAG_NO_CONTROL)) control<false>(c, policy, last);
+      actuation(c);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      make_rows(c);
+      newton(c);
+      add_stats(c);
+      if (last) {
+        post_constraint<true>(c);
+        publish_constraints(c);
+        sync();
+      }
+      if (!(flags & MX_FLAG_NO_INTEGRATE)) {
+        euler(c, damped);
+        if (p.obs.nspec > 0) sample_plan(c);
+      }
+    }
+    if (flags & MX_FLAG_NO_INTEGRATE) break;
+    ++integrated;
+  }
+  if (wave == 0) {
+    publish_derived(c);
+    store_world(c, integrated);
+  }
+}
+
 // The smooth path (models without constraint rows, LDS route) with two wavefronts per world, for
 // batches that leave most wave slots free: wave 0 runs the position stages, then the velocity stage
 // and the mass-matrix inverses while wave 1 runs the FP64 controller up to its bias-free torque
@@ -4962,12 +5029,15 @@ int launch_kernel(const MxModel* m, const MxData* d, const int32_t* mask, int su
 #else
   const size_t shared = p.L.bytes;
 #endif
+#ifdef MX_SLAB
   if (m->njmax > 0)
     hipLaunchKernelGGL(control_step_kernel<true>, dim3(d->nworld), dim3(kLanes), shared, (hipStream_t)stream, p);
   else
-#ifdef MX_SLAB
     hipLaunchKernelGGL(control_step_kernel<false>, dim3(d->nworld), dim3(kLanes), shared, (hipStream_t)stream, p);
 #else
+  if (m->njmax > 0)
+    hipLaunchKernelGGL(control_step_kernel_rows2, dim3(d->nworld), dim3(2 * kLanes), shared, (hipStream_t)stream, p);
+  else
     hipLaunchKernelGGL(control_step_kernel_smooth, dim3(d->nworld), dim3(2 * kLanes), shared, (hipStream_t)stream, p);
 #endif
   return (int)hipGetLastError();
