@@ -1480,8 +1480,8 @@ __device__ void control_bias(const Ctx& c, bool publish) {
 
 // The FP64 OSC proper, on the controller inputs in the O() temporaries (m7, J, q, qd, dbias, eepos,
 // eerot, eevel) and the state in D() (goal, gripper, action, gains, q0, tau); writes tau, ctrl and,
-// at a policy substep, the goal.  C: the step kernel's world context, or the standalone controller
-// kernel's (mx_osc).
+// at a policy substep, the goal.  (mx_osc's kernel, osc_kernel below, computes the same with eight
+// lanes per world.)
 template <bool kSplit, class C>
 __device__ void control_solve(const C& c, int policy, real* ctrl) {
   KModel& m = c.m();
@@ -5236,87 +5236,298 @@ int control_step_noalloc(const MxModel* m, const MxData* d, int substeps, int fl
 struct OscParams {
   MxModel m;
   MxData d;
-  Layout L;
   int flags;
 };
 typedef const __attribute__((address_space(4))) OscParams KOscParams;
 
-// The standalone controller's world context for control_solve(): the controller's doubles (state
-// and temporaries at the layout's double offsets) and its scalar slots in LDS, the model read in
-// place in the kernel argument segment.
-struct OscCtx {
-  KOscParams* p;
-  double* dbl;
-  int* misc;
-  __device__ KModel& m() const { return p->m; }
-  __device__ KLayout& L() const { return p->L; }
-  __device__ int lane() const { return (int)threadIdx.x; }
-  __device__ int* MISC() const { return misc; }
-  __device__ double* O(int off) const { return dbl + off; }
-  __device__ double* D(int off) const { return dbl + off; }
-  __device__ int osc_act(int i) const { return p->m.osc_actuator[i]; }
-  __device__ real ctrlrange(int a, int k) const { return p->m.actuator_ctrlrange[2 * a + k]; }
-};
+// Eight lanes per world, eight worlds per wavefront.  The controller's matrices are at most
+// MX_OSC_MAXDOF wide, so a lane holds a row or a column of each in its registers and a Gauss-Jordan
+// step is one division and a handful of FMAs for all eight worlds; what a lane needs of the others'
+// comes by lane reads, and row owners hand over to column owners through LDS.  (With a wave per world
+// and a lane per matrix entry the kernel was bound by VALU issue, 1195 instructions per world of which
+// most served a few lanes: 16384 worlds took 54.0 us, now 22.1.)  Every value is computed by the operations of
+// control_solve(), in their order.  (The reference's standalone controller kernel, control /
+// control_fast, gpu/cuda/control/osc_solver.cu:309-727, over ControllerSolveData.)  The inputs are the
+// world's published osc_mass, osc_jac, osc_q, osc_qvel, osc_bias and end-effector pose and velocity;
+// the outputs osc_tau, ctrl of the OSC actuators, the goal (policy step), gripper, error and ranks.
+// Groups without a world (the last wave's) run world nworld - 1 along and store nothing: all lanes
+// take part in every lane read.
+constexpr int kOscLanes = 8, kOscWorlds = kLanes / kOscLanes;
+static_assert(MX_OSC_MAXDOF == kOscLanes, "a lane per controlled joint");
+// Doubles per world: the pseudo-inverse fallback's operands, results and work (36 + 2 x 9 each, the
+// work twice), over which the row / column hand-overs (64) lie, then M^-1 J^T.  The stride keeps the
+// eight worlds' LDS banks apart.
+constexpr int kOscMjt = 216, kOscShared = kOscMjt + 6 * MX_OSC_MAXDOF + 2;
 
-// One wavefront per world (the reference's standalone controller kernel, control / control_fast,
-// gpu/cuda/control/osc_solver.cu:309-727, over ControllerSolveData): the inputs are the world's
-// published osc_mass, osc_jac, osc_q, osc_qvel, osc_bias and end-effector pose and velocity; the
-// outputs osc_tau, ctrl of the OSC actuators, the goal (policy step), gripper, error and ranks.
-__global__ __launch_bounds__(kLanes) void osc_kernel(OscParams) {
+__device__ __forceinline__ double lane_double(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_ds_bpermute(lane << 2, (int)b);
+  const int hi = __builtin_amdgcn_ds_bpermute(lane << 2, (int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// One Gauss-Jordan step (gj_inverse()) of the N x N block whose column j this lane holds, its pivot
+// column on lane `owner`; returns whether the pivot is bad.
+template <int N>
+__device__ __forceinline__ bool osc_gj_step(double (&a)[N], int k, int n, int j, int owner) {
+  double col[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) col[i] = i < n ? lane_double(a[i], owner) : 0.0;
+  const double piv = col[k], rowk = (j == k ? 1.0 : a[k]) / piv;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    a[i] = i == k ? rowk : (j == k ? 0.0 : a[i]) - col[i] * rowk;
+  return !(piv > 0.0) || !isfinite(piv);
+}
+
+__global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
   KOscParams* kp = (KOscParams*)__builtin_amdgcn_kernarg_segment_ptr();
-  const int w = blockIdx.x, lane = threadIdx.x;
-  if (w >= kp->d.nworld) return;
   KData& d = kp->d;
-  KLayout& L = kp->L;
-  const size_t ww = (size_t)w;
-  const int nu = kp->m.nu;
-  double* dbl = (double*)mx_lds;
-  int* misc = (int*)(dbl + L.otmp_end);
-  float* ctrl = (float*)(misc + 16);
-  const OscCtx c{kp, dbl, misc};
-  if (lane < 3) dbl[L.goalpos + lane] = d.osc_goal_pos[3 * ww + lane];
-  if (lane < 9) dbl[L.goalrot + lane] = d.osc_goal_rot[9 * ww + lane];
-  if (lane < 2) dbl[L.grip + lane] = d.osc_gripper[2 * ww + lane];
-  const int on = kp->m.osc_ndof;
-  if (lane < 7) dbl[L.action + lane] = lane < 6 ? scaled_action(kp->m, d, ww, lane) : d.osc_action[7 * ww + 6];
-  if (lane < on) {
-    dbl[L.q0 + lane] = d.osc_q0[on * ww + lane];
-    dbl[L.tau + lane] = d.osc_tau[on * ww + lane];
-    dbl[L.q + lane] = d.osc_q[on * ww + lane];
-    dbl[L.qd + lane] = d.osc_qvel[on * ww + lane];
-    dbl[L.dbias + lane] = d.osc_bias[on * ww + lane];
+  KModel& m = kp->m;
+  constexpr int N = MX_OSC_MAXDOF;
+  __shared__ double shared[kOscWorlds * kOscShared];
+  const int lane = threadIdx.x, group = lane / kOscLanes, g0 = group * kOscLanes, j = lane % kOscLanes;
+  const int world = (int)blockIdx.x * kOscWorlds + group;
+  const bool have = world < d.nworld;
+  const size_t w = have ? world : d.nworld - 1;
+  double* X = shared + group * kOscShared;
+  double* mjt = X + kOscMjt;
+  const int on = m.osc_ndof, nu = m.nu;
+  const int jn = j < on ? j : 0, j6 = j < 6 ? j : 0;   // clamped for loads
+  const bool policy = kp->flags & MX_FLAG_POLICY_FIRST;
+  bool live = have && d.osc_error[w] == 0;
+
+  // inputs: column j and row j of M, all of J
+  double a[N], mrow[N], J[6][N], minv[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int q = i < on ? i : 0;
+    a[i] = i < on && j < on ? (double)d.osc_mass[on * on * w + q * on + jn] : 0.0;
+    mrow[i] = d.osc_mass[on * on * w + jn * on + q];
+#pragma unroll
+    for (int r = 0; r < 6; ++r) J[r][i] = i < on ? (double)d.osc_jac[6 * on * w + r * on + q] : 0.0;
   }
-  if (lane < 12) dbl[L.gains + lane] = d.osc_gains[12 * ww + lane];
-  if (lane < on * on) dbl[L.m7 + lane] = d.osc_mass[on * on * ww + lane];
-  if (lane < 6 * on) dbl[L.J + lane] = d.osc_jac[6 * on * ww + lane];
-  if (lane < 3) dbl[L.eepos + lane] = d.osc_ee_pos[3 * ww + lane];
-  if (lane < 9) dbl[L.eerot + lane] = d.osc_ee_rot[9 * ww + lane];
-  if (lane < 6) dbl[L.eevel + lane] = d.osc_ee_vel[6 * ww + lane];
-  for (int a = lane; a < nu; a += kLanes) ctrl[a] = d.ctrl[ww * nu + a];
-  if (lane < 16) misc[lane] = 0;
+  double eep[3], eer[9];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) eep[k] = d.osc_ee_pos[3 * w + k];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) eer[k] = d.osc_ee_rot[9 * w + k];
+  const double bias = d.osc_bias[on * w + jn];
+  const double pdj = 10.0 * (d.osc_q0[on * w + jn] - (double)d.osc_q[on * w + jn]) -
+                     6.324555320336759 * (double)d.osc_qvel[on * w + jn];
+  const double ev = d.osc_ee_vel[6 * w + j6], kpj = d.osc_gains[12 * w + j6], kdj = d.osc_gains[12 * w + 6 + j6];
+
+  // M^-1
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (k < on) bad |= osc_gj_step(a, k, on, j, g0 + k);
+  if (live && bad) {
+    live = false;
+    if (j == 0) d.osc_error[w] = MX_OSC_SINGULAR_MASS;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) X[i * N + j] = a[i];
   sync();
-  if (lane == 0) {
-    misc[kCtrlErr] = d.osc_error[ww];
-    for (int k = 0; k < 3; ++k) misc[kRank0 + k] = d.osc_rank[3 * ww + k];
+#pragma unroll
+  for (int k = 0; k < N; ++k) minv[k] = X[j * N + k];
+  sync();
+
+  // M^-1 J^T: row j here, to all lanes through LDS (n x 6)
+#pragma unroll
+  for (int col = 0; col < 6; ++col) {
+    double s = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (k < on) s += minv[k] * J[col][k];
+    mjt[j * 6 + col] = s;
   }
   sync();
-  control_solve<false>(c, kp->flags & MX_FLAG_POLICY_FIRST, ctrl);
+
+  // A = J M^-1 J^T, column j < 6; b: its column of A_pos (j < 3) or A_ori
+  double A[6], b[3], Af[6], bf[3];
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    double s = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (k < on) s += J[r][k] * mjt[k * 6 + j6];
+    A[r] = Af[r] = j < 6 ? s : 0.0;
+  }
+  const int half = j < 3 ? 0 : 3, jl = j - half;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) b[r] = bf[r] = half ? A[3 + r] : A[r];
+  bool bada = false, badb = false;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) bada |= osc_gj_step(Af, k, 6, j, g0 + k);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) badb |= osc_gj_step(bf, k, 3, jl, g0 + half + k);
+
+  // whether each inverse is the pseudo-inverse (traces); else the fallback, a lane per operand
+  double ta[3] = {0, 0, 0}, ti[3] = {0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    ta[0] += lane_double(A[k], g0 + k);
+    ti[0] += lane_double(Af[k], g0 + k);
+    ta[1 + k / 3] += lane_double(b[k % 3], g0 + k);
+    ti[1 + k / 3] += lane_double(bf[k % 3], g0 + k);
+  }
+  const unsigned int badg = (unsigned int)(__ballot(badb) >> g0);   // lanes 0 (A_pos) and 3 (A_ori)
+  const bool fast0 = !bada && ti[0] > 0 && ta[0] * ti[0] <= 1e13;
+  const bool fast1 = !(badg & 1u) && ti[1] > 0 && ta[1] * ti[1] <= 1e13;
+  const bool fast2 = !(badg & 8u) && ti[2] > 0 && ta[2] * ti[2] <= 1e13;
+  if (__any(live && !(fast0 && fast1 && fast2))) {
+    double* src = X;          // A, A_pos, A_ori
+    double* inv = X + 54;     // their pseudo-inverses
+    double* work = X + 108;   // 72 + 18 + 18
+    if (j < 6) {
+#pragma unroll
+      for (int r = 0; r < 6; ++r) src[r * 6 + j] = A[r];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) src[36 + 3 * half + r * 3 + jl] = b[r];
+    }
+    sync();
+    const bool slow = live && (j == 0 ? !fast0 : (j == 1 ? !fast1 : (j == 2 && !fast2)));
+    int rank = j == 0 ? 6 : 3, ok = 1;
+    if (slow) {
+      const int n = j == 0 ? 6 : 3, at = j == 0 ? 0 : 27 + 9 * j;
+      double* wk = work + (j == 0 ? 0 : 54 + 18 * j);
+      ok = jacobi_pinv(src + at, n, inv + at, &rank, wk, wk + n * n);
+    }
+    sync();
+    if (live && j < 3) d.osc_rank[3 * w + j] = rank;
+    if (!fast0)
+#pragma unroll
+      for (int r = 0; r < 6; ++r) Af[r] = inv[r * 6 + j6];
+    if (half ? !fast2 : !fast1)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) bf[r] = inv[36 + 3 * half + r * 3 + (j < 6 ? jl : 0)];
+    sync();
+    const unsigned int failed = (unsigned int)(__ballot(!ok) >> g0) & 7u;
+    if (live && failed) {
+      live = false;
+      if (j == 0) d.osc_error[w] = MX_OSC_PINV_FAILED;
+    }
+  } else if (live && j < 3) {
+    d.osc_rank[3 * w + j] = j == 0 ? 6 : 3;
+  }
+
+  // J-bar = M^-1 J^T Lambda (n x 6), column j here, to all lanes through LDS
+  if (j < 6) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      double s = 0;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) s += mjt[i * 6 + k] * Af[k];
+      X[i * 6 + j] = s;
+    }
+  }
   sync();
-  if (lane < on) d.osc_tau[on * ww + lane] = dbl[L.tau + lane];
-  if (lane < 3) d.osc_goal_pos[3 * ww + lane] = dbl[L.goalpos + lane];
-  if (lane < 9) d.osc_goal_rot[9 * ww + lane] = dbl[L.goalrot + lane];
-  if (lane < 2) d.osc_gripper[2 * ww + lane] = dbl[L.grip + lane];
-  if (lane < 3) d.osc_rank[3 * ww + lane] = misc[kRank0 + lane];
-  if (lane == 0) d.osc_error[ww] = misc[kCtrlErr];
-  for (int a = lane; a < nu; a += kLanes) d.ctrl[ww * nu + a] = ctrl[a];
+
+  // the goal (every lane of the world computes it)
+  double gp[3], gr[9];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) gp[k] = d.osc_goal_pos[3 * w + k];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) gr[k] = d.osc_goal_rot[9 * w + k];
+  if (policy) {
+    const double mine = scaled_action(m, d, w, j6);
+    double action[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) action[k] = lane_double(mine, g0 + k);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) gp[k] = eep[k] + action[k];
+    if (action[3] != 0.0 || action[4] != 0.0 || action[5] != 0.0) {
+      double R[9];
+      rotation_delta(action[3], action[4], action[5], R);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          gr[3 * i + q] = R[3 * i] * eer[q] + R[3 * i + 1] * eer[3 + q] + R[3 * i + 2] * eer[6 + q];
+    }
+    if (live && j == 0) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d.osc_goal_pos[3 * w + k] = gp[k];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) d.osc_goal_rot[9 * w + k] = gr[k];
+    }
+  }
+
+  // desired acceleration j (position 0-2, orientation 3-5) and the wrench
+  double er[3], ep[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int nx = (r + 1) % 3, ls = (r + 2) % 3;
+    er[r] = 0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) er[r] += 0.5 * (eer[nx * 3 + q] * gr[ls * 3 + q] - eer[ls * 3 + q] * gr[nx * 3 + q]);
+    ep[r] = gp[r] - eep[r];
+  }
+  const double e3 = jl == 0 ? (half ? er[0] : ep[0]) : (jl == 1 ? (half ? er[1] : ep[1]) : (half ? er[2] : ep[2]));
+  const double desired = kpj * e3 - kdj * ev;
+  double wrench[6] = {0, 0, 0, 0, 0, 0};
+  // (the sum over k runs through the columns' owners: lane k holds column k of Lambda)
+  if (m.osc_uncouple) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const double x = lane_double(desired, g0 + k);
+#pragma unroll
+      for (int r = 0; r < 3; ++r) wrench[k / 3 * 3 + r] += lane_double(bf[r], g0 + k) * x;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const double x = lane_double(desired, g0 + k);
+#pragma unroll
+      for (int r = 0; r < 6; ++r) wrench[r] += lane_double(Af[r], g0 + k) * x;
+    }
+  }
+
+  // posture torque j, the nullspace column j of N = I - J-bar J, and the torque
+  double posture = 0, task = 0, null = 0, Jj[6];
+#pragma unroll
+  for (int r = 0; r < 6; ++r) Jj[r] = d.osc_jac[6 * on * w + r * on + jn];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const double pd = lane_double(pdj, g0 + k);
+    if (k < on) posture += mrow[k] * pd;
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) task += Jj[k] * wrench[k];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const double p = lane_double(posture, g0 + i);
+    double s = 0;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s += X[i * 6 + k] * Jj[k];
+    if (i < on) null += ((i == j ? 1.0 : 0.0) - s) * p;
+  }
+  if (!live) return;
+  if (j < on) {
+    const double t = task + bias + null;
+    d.osc_tau[on * w + j] = t;
+    const int act = m.osc_actuator[j];
+    const double lo = m.actuator_ctrlrange[2 * act], hi = m.actuator_ctrlrange[2 * act + 1];
+    d.ctrl[w * nu + act] = (real)(isnan(t) ? t : fmin(hi, fmax(lo, t)));
+  }
+  if (j < 2) {   // gripper actuator j
+    const double a6 = d.osc_action[7 * w + 6];
+    const double sgn = isnan(a6) ? a6 : (a6 > 0 ? 1.0 : (a6 < 0 ? -1.0 : 0.0));
+    const double v = clip1(d.osc_gripper[2 * w + j] + (double)m.osc_gripper_speed * (j == 0 ? -1.0 : 1.0) * sgn);
+    d.osc_gripper[2 * w + j] = v;
+    const int act = m.osc_actuator[on + j];
+    const double lo = m.actuator_ctrlrange[2 * act], hi = m.actuator_ctrlrange[2 * act + 1];
+    d.ctrl[w * nu + act] = (real)((hi + lo) * 0.5 + (hi - lo) * 0.5 * v);
+  }
 }
 
 int osc_launch(const MxModel* m, const MxData* d, int flags, void* stream) {
   const int rc = mx_check(m, d);
   if (rc) return rc;
-  const OscParams a{*m, *d, make_layout(*m), flags};
-  const size_t shared = (size_t)a.L.otmp_end * sizeof(double) + 16 * sizeof(int) + (size_t)m->nu * sizeof(float);
-  hipLaunchKernelGGL(osc_kernel, dim3(d->nworld), dim3(kLanes), shared, (hipStream_t)stream, a);
+  const OscParams a{*m, *d, flags};
+  const int blocks = d->nworld / kOscWorlds + (d->nworld % kOscWorlds != 0);
+  hipLaunchKernelGGL(osc_kernel, dim3(blocks), dim3(kLanes), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
 
