@@ -5245,7 +5245,7 @@ typedef const __attribute__((address_space(4))) OscParams KOscParams;
 // step is one division and a handful of FMAs for all eight worlds; what a lane needs of the others'
 // comes by lane reads, and row owners hand over to column owners through LDS.  (With a wave per world
 // and a lane per matrix entry the kernel was bound by VALU issue, 1195 instructions per world of which
-// most served a few lanes: 16384 worlds took 54.0 us, now 22.1.)  Every value is computed by the operations of
+// most served a few lanes: 16384 worlds took 54.0 us, now 18.1; 16 worlds 14.0, now 10.3.)  Every value is computed by the operations of
 // control_solve(), in their order.  (The reference's standalone controller kernel, control /
 // control_fast, gpu/cuda/control/osc_solver.cu:309-727, over ControllerSolveData.)  The inputs are the
 // world's published osc_mass, osc_jac, osc_q, osc_qvel, osc_bias and end-effector pose and velocity;
@@ -5255,7 +5255,7 @@ typedef const __attribute__((address_space(4))) OscParams KOscParams;
 constexpr int kOscLanes = 8, kOscWorlds = kLanes / kOscLanes;
 static_assert(MX_OSC_MAXDOF == kOscLanes, "a lane per controlled joint");
 // Doubles per world: the pseudo-inverse fallback's operands, results and work (36 + 2 x 9 each, the
-// work twice), over which the row / column hand-overs (64) lie, then M^-1 J^T.  The stride keeps the
+// work twice), over which the row / column hand-overs (64) and J (48) lie, then M^-1 J^T.  The stride keeps the
 // eight worlds' LDS banks apart.
 constexpr int kOscMjt = 216, kOscShared = kOscMjt + 6 * MX_OSC_MAXDOF + 2;
 
@@ -5266,18 +5266,30 @@ __device__ __forceinline__ double lane_double(double v, int lane) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// One Gauss-Jordan step (gj_inverse()) of the N x N block whose column j this lane holds, its pivot
-// column on lane `owner`; returns whether the pivot is bad.
+// Gauss-Jordan inversion (gj_inverse()) of the n x n block whose column j this lane holds, column k on
+// lane owner + k; returns whether a pivot was bad.  Rows from n on are zero and stay so.  The rows
+// rotate by one per step, so the pivot row is always the first register and the step stays one loop
+// body: a small batch waits for the kernel's instructions more than for anything
+// else (unrolled, with J loaded whole by every lane, 31 KB of code: 16 worlds 15.9 us instead of 10.3,
+// 16384 22.1 instead of 18.1).
 template <int N>
-__device__ __forceinline__ bool osc_gj_step(double (&a)[N], int k, int n, int j, int owner) {
-  double col[N];
+__device__ __forceinline__ bool osc_gj(double (&a)[N], int n, int j, int owner) {
+  bool bad = false;
+#pragma unroll 1
+  for (int k = 0; k < n; ++k) {
+    double col[N];
 #pragma unroll
-  for (int i = 0; i < N; ++i) col[i] = i < n ? lane_double(a[i], owner) : 0.0;
-  const double piv = col[k], rowk = (j == k ? 1.0 : a[k]) / piv;
+    for (int i = 0; i < N; ++i) col[i] = lane_double(a[i], owner + k);
+    const double piv = col[0], rowk = (j == k ? 1.0 : a[0]) / piv;
+    bad |= !(piv > 0.0) || !isfinite(piv);
 #pragma unroll
-  for (int i = 0; i < N; ++i)
-    a[i] = i == k ? rowk : (j == k ? 0.0 : a[i]) - col[i] * rowk;
-  return !(piv > 0.0) || !isfinite(piv);
+    for (int i = 0; i + 1 < N; ++i) {
+      const double next = (j == k ? 0.0 : a[i + 1]) - col[i + 1] * rowk;
+      a[i] = i == n - 1 ? rowk : next;
+    }
+    a[N - 1] = n == N ? rowk : 0.0;
+  }
+  return bad;
 }
 
 __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
@@ -5297,16 +5309,19 @@ __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
   const bool policy = kp->flags & MX_FLAG_POLICY_FIRST;
   bool live = have && d.osc_error[w] == 0;
 
-  // inputs: column j and row j of M, all of J
-  double a[N], mrow[N], J[6][N], minv[N];
+  // inputs: column j and row j of M, column j of J (all of J through LDS); zero past the joints
+  double a[N], mrow[N], Jj[6], J[6][N];
+  const float* gm = d.osc_mass + on * on * w;
+  const float* gj = d.osc_jac + 6 * on * w;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const int q = i < on ? i : 0;
-    a[i] = i < on && j < on ? (double)d.osc_mass[on * on * w + q * on + jn] : 0.0;
-    mrow[i] = d.osc_mass[on * on * w + jn * on + q];
-#pragma unroll
-    for (int r = 0; r < 6; ++r) J[r][i] = i < on ? (double)d.osc_jac[6 * on * w + r * on + q] : 0.0;
+    const float x = gm[q * on + jn], y = gm[jn * on + q];
+    a[i] = i < on && j < on ? (double)x : 0.0;
+    mrow[i] = i < on ? (double)y : 0.0;
   }
+#pragma unroll
+  for (int r = 0; r < 6; ++r) Jj[r] = j < on ? (double)gj[r * on + jn] : 0.0;
   double eep[3], eer[9];
 #pragma unroll
   for (int k = 0; k < 3; ++k) eep[k] = d.osc_ee_pos[3 * w + k];
@@ -5318,28 +5333,30 @@ __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
   const double ev = d.osc_ee_vel[6 * w + j6], kpj = d.osc_gains[12 * w + j6], kdj = d.osc_gains[12 * w + 6 + j6];
 
   // M^-1
-  bool bad = false;
-#pragma unroll
-  for (int k = 0; k < N; ++k)
-    if (k < on) bad |= osc_gj_step(a, k, on, j, g0 + k);
+  const bool bad = osc_gj(a, on, j, g0);
   if (live && bad) {
     live = false;
     if (j == 0) d.osc_error[w] = MX_OSC_SINGULAR_MASS;
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) X[i * N + j] = a[i];
+#pragma unroll
+  for (int r = 0; r < 6; ++r) X[N * N + r * N + j] = Jj[r];
   sync();
+  double minv[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) minv[k] = X[j * N + k];
-  sync();
+#pragma unroll
+  for (int r = 0; r < 6; ++r)
+#pragma unroll
+    for (int k = 0; k < N; ++k) J[r][k] = X[N * N + r * N + k];
 
   // M^-1 J^T: row j here, to all lanes through LDS (n x 6)
 #pragma unroll
   for (int col = 0; col < 6; ++col) {
     double s = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k)
-      if (k < on) s += minv[k] * J[col][k];
+    for (int k = 0; k < N; ++k) s += minv[k] * J[col][k];
     mjt[j * 6 + col] = s;
   }
   sync();
@@ -5350,26 +5367,23 @@ __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
   for (int r = 0; r < 6; ++r) {
     double s = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k)
-      if (k < on) s += J[r][k] * mjt[k * 6 + j6];
+    for (int k = 0; k < N; ++k) s += J[r][k] * mjt[k * 6 + j6];
     A[r] = Af[r] = j < 6 ? s : 0.0;
   }
   const int half = j < 3 ? 0 : 3, jl = j - half;
 #pragma unroll
   for (int r = 0; r < 3; ++r) b[r] = bf[r] = half ? A[3 + r] : A[r];
-  bool bada = false, badb = false;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) bada |= osc_gj_step(Af, k, 6, j, g0 + k);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) badb |= osc_gj_step(bf, k, 3, jl, g0 + half + k);
+  const bool bada = osc_gj(Af, 6, j, g0);
+  const bool badb = osc_gj(bf, 3, jl, g0 + half);
 
   // whether each inverse is the pseudo-inverse (traces); else the fallback, a lane per operand
   double ta[3] = {0, 0, 0}, ti[3] = {0, 0, 0};
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
-    ta[0] += lane_double(A[k], g0 + k);
+    const double diag = lane_double(A[k], g0 + k);   // A_pos's and A_ori's too
+    ta[0] += diag;
     ti[0] += lane_double(Af[k], g0 + k);
-    ta[1 + k / 3] += lane_double(b[k % 3], g0 + k);
+    ta[1 + k / 3] += diag;
     ti[1 + k / 3] += lane_double(bf[k % 3], g0 + k);
   }
   const unsigned int badg = (unsigned int)(__ballot(badb) >> g0);   // lanes 0 (A_pos) and 3 (A_ori)
@@ -5485,23 +5499,18 @@ __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
   }
 
   // posture torque j, the nullspace column j of N = I - J-bar J, and the torque
-  double posture = 0, task = 0, null = 0, Jj[6];
+  double posture = 0, task = 0, null = 0;
 #pragma unroll
-  for (int r = 0; r < 6; ++r) Jj[r] = d.osc_jac[6 * on * w + r * on + jn];
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const double pd = lane_double(pdj, g0 + k);
-    if (k < on) posture += mrow[k] * pd;
-  }
+  for (int k = 0; k < N; ++k) posture += mrow[k] * lane_double(pdj, g0 + k);
+  if (j >= on) posture = 0;
 #pragma unroll
   for (int k = 0; k < 6; ++k) task += Jj[k] * wrench[k];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const double p = lane_double(posture, g0 + i);
     double s = 0;
 #pragma unroll
     for (int k = 0; k < 6; ++k) s += X[i * 6 + k] * Jj[k];
-    if (i < on) null += ((i == j ? 1.0 : 0.0) - s) * p;
+    null += ((i == j ? 1.0 : 0.0) - s) * lane_double(posture, g0 + i);
   }
   if (!live) return;
   if (j < on) {
