@@ -75,12 +75,19 @@ __host__ __device__ inline Image image_layout(const MxModel& m) {
   return I;
 }
 
-// Copy the model arrays into the image (all lanes of the wavefront cooperate).
+// Copy the model arrays into the image: by `lanes` threads, all parts (one wavefront of the LDS route),
+// or part `part` of kImageParts by thread `lane` of workgroup `block` of `blocks` such groups.  No word
+// depends on another.
+constexpr int kImageParts = 11;
 // m and I are read in place in the kernel argument segment.
 __device__ inline void stage_image(KModel& m, const __attribute__((address_space(4))) Image& I, float* f, int lane,
-                                   int lanes) {
+                                   int lanes, int part = -1, int block = 0, int blocks = 1) {
   int* n = reinterpret_cast<int*>(f);
-  for (int t = lane; t < m.nbody * BR; t += lanes) {
+  const int thread = lane, threads = lanes;
+  lane += block * threads;
+  lanes *= blocks;
+  auto mine = [&](int k) { return part < 0 || part == k; };
+  if (mine(0)) for (int t = lane; t < m.nbody * BR; t += lanes) {
     int b = t / BR, k = t % BR;
     float* rf = f + I.body + BR * b;
     int* ri = n + I.body + BR * b;
@@ -106,7 +113,7 @@ __device__ inline void stage_image(KModel& m, const __attribute__((address_space
         else rf[k] = m.body_invweight0[2 * b + k - B_INVW];
     }
   }
-  for (int t = lane; t < m.njnt * JR; t += lanes) {
+  if (mine(1)) for (int t = lane; t < m.njnt * JR; t += lanes) {
     int j = t / JR, k = t % JR;
     float* rf = f + I.jnt + JR * j;
     int* ri = n + I.jnt + JR * j;
@@ -129,7 +136,7 @@ __device__ inline void stage_image(KModel& m, const __attribute__((address_space
         else rf[k] = m.jnt_solimp[5 * j + k - J_SOLIMP];
     }
   }
-  for (int t = lane; t < m.nv * DR; t += lanes) {
+  if (mine(2)) for (int t = lane; t < m.nv * DR; t += lanes) {
     int d = t / DR, k = t % DR;
     float* rf = f + I.dof + DR * d;
     int* ri = n + I.dof + DR * d;
@@ -147,7 +154,7 @@ __device__ inline void stage_image(KModel& m, const __attribute__((address_space
         else rf[k] = m.dof_solimp[5 * d + k - D_SOLIMP];
     }
   }
-  for (int t = lane; t < m.ngeom * GR; t += lanes) {
+  if (mine(3)) for (int t = lane; t < m.ngeom * GR; t += lanes) {
     int g = t / GR, k = t % GR;
     float* rf = f + I.geom + GR * g;
     int* ri = n + I.geom + GR * g;
@@ -173,13 +180,13 @@ __device__ inline void stage_image(KModel& m, const __attribute__((address_space
         else rf[k] = m.geom_solimp[5 * g + k - G_SOLIMP];
     }
   }
-  for (int t = lane; t < m.nsite * SR; t += lanes) {
+  if (mine(4)) for (int t = lane; t < m.nsite * SR; t += lanes) {
     int s = t / SR, k = t % SR;
     if (k == S_BODY) n[I.site + SR * s + k] = m.site_body[s];
     else if (k < S_QUAT) f[I.site + SR * s + k] = m.site_pos[3 * s + k - S_POS];
     else f[I.site + SR * s + k] = m.site_quat[4 * s + k - S_QUAT];
   }
-  for (int t = lane; t < m.nu * AR; t += lanes) {
+  if (mine(4)) for (int t = lane; t < m.nu * AR; t += lanes) {
     int a = t / AR, k = t % AR;
     float* rf = f + I.act + AR * a;
     int* ri = n + I.act + AR * a;
@@ -198,45 +205,47 @@ __device__ inline void stage_image(KModel& m, const __attribute__((address_space
         else rf[k] = m.actuator_forcerange[2 * a + k - A_FORCERANGE];
     }
   }
-  for (int t = lane; t < m.ntree * TR; t += lanes) {
+  if (mine(5)) for (int t = lane; t < m.ntree * TR; t += lanes) {
     int tr = t / TR, k = t % TR;
     n[I.tree + t] = k == T_DOFADR ? m.tree_dofadr[tr] : (k == T_DOFNUM ? m.tree_dofnum[tr] :
                     (k == T_MADR ? m.tree_madr[tr] : (m.tree_dampadr[tr] < 0 ? -1 : m.nM + m.tree_dampadr[tr])));
   }
-  for (int t = lane; t < m.nMpair; t += lanes) {
+  if (mine(5)) for (int t = lane; t < m.nMpair; t += lanes) {
     n[I.mpair + 2 * t] = m.mpair_i[t];
     n[I.mpair + 2 * t + 1] = m.mpair_j[t];
   }
   // mass-block entry -> block address (10 bits), size (6), row (6), column (6); then the row's dof.
   // The damped blocks of damped trees follow the nM mass entries.
-  for (int tr = 0; tr < m.ntree; ++tr) {
+  if (mine(6)) for (int tr = block; tr < m.ntree; tr += blocks) {
     int nn = m.tree_dofnum[tr];
     for (int pass = 0; pass < 2; ++pass) {
       if (pass == 1 && m.tree_dampadr[tr] < 0) break;
       int adr = pass == 0 ? m.tree_madr[tr] : m.nM + m.tree_dampadr[tr];
-      for (int e = lane; e < nn * nn; e += lanes) {
+      for (int e = thread; e < nn * nn; e += threads) {
         n[I.mentry + 2 * (adr + e)] = adr | (nn << 10) | ((e / nn) << 16) | ((e % nn) << 22);
         n[I.mentry + 2 * (adr + e) + 1] = m.tree_dofadr[tr] + e / nn;
       }
     }
   }
-  for (int b = lane; b < m.nbody; b += lanes) {
+  if (mine(7)) for (int b = lane; b < m.nbody; b += lanes) {
     int* ch = n + I.chain + I.chainw * b;
     int cnt = 0;
     for (int dd = m.body_lastdof[b]; dd >= 0; dd = m.dof_parent[dd]) ch[1 + cnt++] = dd;
     ch[0] = cnt;
   }
-  for (int t = lane; t < m.nlevel + 1; t += lanes) n[I.level + t] = m.level_adr[t];
-  for (int t = lane; t < m.nbody - 1; t += lanes) n[I.level + m.nlevel + 1 + t] = m.level_body[t];
-  if (lane < m.osc_ndof) {
-    n[I.osc + lane] = m.osc_qposadr[lane];
-    n[I.osc + MX_OSC_MAXDOF + lane] = m.osc_dofadr[lane];
+  if (mine(8)) {
+    for (int t = lane; t < m.nlevel + 1; t += lanes) n[I.level + t] = m.level_adr[t];
+    for (int t = lane; t < m.nbody - 1; t += lanes) n[I.level + m.nlevel + 1 + t] = m.level_body[t];
+    if (lane < m.osc_ndof) {
+      n[I.osc + lane] = m.osc_qposadr[lane];
+      n[I.osc + MX_OSC_MAXDOF + lane] = m.osc_dofadr[lane];
+    }
+    if (lane < m.osc_ndof + 2) n[I.osc + 2 * MX_OSC_MAXDOF + lane] = m.osc_actuator[lane];
   }
-  if (lane < m.osc_ndof + 2) n[I.osc + 2 * MX_OSC_MAXDOF + lane] = m.osc_actuator[lane];
   if (m.njmax > 0) {
-    for (int t = lane; t < 2 * m.npair; t += lanes) n[I.pair + t] = m.pair_geom[t];
-    for (int t = lane; t < 4 * m.nmeshvert; t += lanes) f[I.mesh + t] = (t & 3) == 3 ? 0.f : m.mesh_vert[3 * (t >> 2) + (t & 3)];
-    for (int t = lane; t < m.nmesh; t += lanes) {
+    if (mine(9)) for (int t = lane; t < 2 * m.npair; t += lanes) n[I.pair + t] = m.pair_geom[t];
+    if (mine(10)) for (int t = lane; t < 4 * m.nmeshvert; t += lanes) f[I.mesh + t] = (t & 3) == 3 ? 0.f : m.mesh_vert[3 * (t >> 2) + (t & 3)];
+    if (mine(8)) for (int t = lane; t < m.nmesh; t += lanes) {
       n[I.meshrec + 2 * t] = m.mesh_vertadr[t];
       n[I.meshrec + 2 * t + 1] = m.mesh_vertnum[t];
     }
