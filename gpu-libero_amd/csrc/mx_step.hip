@@ -274,9 +274,9 @@ Layout make_layout(const MxModel& m) {
     const int need_rows = 7 * m.nv + 3 * m.nbody + (m.maxchain + 1) * m.nbody;
     if (m.njmax > 0 && L.win < need_rows) L.win = round_up(need_rows, 4);
   }
-  // the islands' tables (islands(): 8 ntree + 2 words, two per contact and two per dof)
-  if (m.njmax > 0 && L.win < 8 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv)
-    L.win = round_up(8 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv, 4);
+  // the islands' tables (islands(): 7 ntree + 2 words, two per contact and two per dof)
+  if (m.njmax > 0 && L.win < 7 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv)
+    L.win = round_up(7 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv, 4);
   // the geoms' collision records after the EPA block
   if (m.njmax > 0 && L.win < L.gpose + GP_WORDS * m.ngeom) L.win = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
   // then the hull vertices (4 words each), read by every support-point search of the stage
@@ -2845,10 +2845,7 @@ __device__ __forceinline__ int hdecode(const IP* iblk, int nisl, int e, int tota
 }
 
 // Islands: trees joined by contact rows (union-find by one lane).  Each island's Hessian is a
-// dense block (packed lower triangle); trees in island order, dofs of a tree consecutive.  A tree
-// without a row (no contact, limit or friction row touches it: most often the arm, and every parked
-// object) belongs to no island (disl -1): its Hessian is its mass block, so its part of every Newton
-// step is known without one (FreeTrees below).
+// dense block (packed lower triangle); trees in island order, dofs of a tree consecutive.
 __device__ void islands(const Ctx& c) {
   KModel& m = c.m();
   int* sv = c.SV();
@@ -2873,9 +2870,7 @@ __device__ void islands(const Ctx& c) {
   sint* ctr = listart + nt + 1;   // each contact's two trees (-1: contact without rows)
   sint* ldisl = ctr + 2 * ncon;   // dof -> island, island-local index
   sint* ldloc = ldisl + m.nv;
-  sint* touched = ldloc + m.nv;   // nt: whether a row touches the tree
-  for (int t = c.lane(); t < nt; t += kLanes) { uf[t] = t; tdn[t] = c.ti(t, T_DOFNUM); touched[t] = 0; }
-  sync();
+  for (int t = c.lane(); t < nt; t += kLanes) { uf[t] = t; tdn[t] = c.ti(t, T_DOFNUM); }
   for (int con = c.lane(); con < ncon; con += kLanes) {
     int t1 = -1, t2 = -1;
     if (c.N(c.L().caddr)[con] >= 0) {
@@ -2884,24 +2879,14 @@ __device__ void islands(const Ctx& c) {
     }
     ctr[2 * con] = t1;
     ctr[2 * con + 1] = t2;
-    if (t1 >= 0) touched[t1] = 1;
-    if (t2 >= 0) touched[t2] = 1;
-  }
-  const int nsingle = min(sv[SV_NF] + sv[SV_NL], sv[SV_NEFC]);   // single-dof rows come first
-  for (int r = c.lane(); r < nsingle; r += kLanes) {
-    real sign;
-    int kind;
-    touched[c.di(single_dof(c.N(c.L().rid)[r], sign, kind), D_TREE)] = 1;
   }
   sync();
-  // Every table below is a function of this list and of the touched trees alone (the union-find's
-  // partition of the trees, the tree order numbering the islands): when each contact joins the same
-  // two trees as in the substep the tables were built for (same count and order, kept in ctrp) and
-  // the same trees are touched, they still hold.
+  // Every table below is a function of this list alone (the union-find's partition of the trees,
+  // the tree order numbering the islands): when each contact joins the same two trees as in the
+  // substep the tables were built for (same count and order, kept in ctrp), they still hold.
   int* prev = c.N(c.L().ctrp);
   if (sv[SV_ISLAND]) {
     bool diff = prev[0] != ncon;
-    for (int t = c.lane(); t < nt; t += kLanes) diff |= (tisl[t] >= 0) != (touched[t] != 0);
     for (int t = c.lane(); t < 2 * ncon; t += kLanes) diff |= prev[1 + t] != ctr[t];
     if (!__any(diff)) return;
   }
@@ -2922,13 +2907,11 @@ __device__ void islands(const Ctx& c) {
     int nisl = 0;
     for (int t = 0; t < nt; ++t) {
       int r = find(t);
-      ltisl[t] = !touched[t] ? -1 : (r == t ? nisl++ : ltisl[r]);
+      ltisl[t] = r == t ? nisl++ : ltisl[r];
     }
     for (int i = 0; i < nisl; ++i) lisz[i] = 0;
     for (int t = 0; t < nt; ++t) {
       int I = ltisl[t];
-      ltoff[t] = 0;
-      if (I < 0) continue;
       ltoff[t] = lisz[I];
       lisz[I] += tdn[t];
     }
@@ -2957,7 +2940,7 @@ __device__ void islands(const Ctx& c) {
     c.N(c.L().dloc)[d] = li;
     ldisl[d] = I;
     ldloc[d] = li;
-    if (I >= 0) c.N(c.L().idof)[listart[I] + li] = d;
+    c.N(c.L().idof)[listart[I] + li] = d;
   }
   sync();
   // the Hessian assembly's mass-entry map and the sweep's per-lane decodes, from the LDS tables:
@@ -2967,7 +2950,7 @@ __device__ void islands(const Ctx& c) {
   for (int e = c.lane(); e < m.nM; e += kLanes) {
     int cd = ent[2 * e], i = (cd >> 16) & 63, j = (cd >> 22) & 63;
     int di = ent[2 * e + 1], dj = di - i + j, li = ldloc[di];
-    hmap[e] = j > i || ldisl[di] < 0 ? -1 : liblk[ldisl[di]] + li * (li + 1) / 2 + ldloc[dj];
+    hmap[e] = j > i ? -1 : liblk[ldisl[di]] + li * (li + 1) / 2 + ldloc[dj];
   }
   const int total = liblk[nisl];
   int* own = c.N(c.L().hown);
@@ -2979,7 +2962,7 @@ __device__ void islands(const Ctx& c) {
     own[(2 * kOwn + q) * kLanes + c.lane()] = code >= 0 ? listart[I] : 0;
   }
   int sn[4] = {0, 0, 0, 0};
-  if (c.lane() < m.nv && ldisl[c.lane()] >= 0) {
+  if (c.lane() < m.nv) {
     int I = ldisl[c.lane()];
     sn[0] = lisz[I]; sn[1] = listart[I] + ldloc[c.lane()]; sn[2] = ldloc[c.lane()]; sn[3] = liblk[I];
   }
@@ -2988,23 +2971,14 @@ __device__ void islands(const Ctx& c) {
   sync();
 #else
   if (c.lane() == 0) {
-    int* uf = iblk;        // scratch: parent pointers
-    int* touched = toff;   // scratch: whether a row touches the tree
-    for (int t = 0; t < nt; ++t) { uf[t] = t; touched[t] = 0; }
-    const int nsingle = min(sv[SV_NF] + sv[SV_NL], sv[SV_NEFC]);   // single-dof rows come first
-    for (int r = 0; r < nsingle; ++r) {
-      real sign;
-      int kind;
-      touched[c.di(single_dof(c.N(c.L().rid)[r], sign, kind), D_TREE)] = 1;
-    }
+    int* uf = iblk;   // scratch: parent pointers
+    for (int t = 0; t < nt; ++t) uf[t] = t;
     auto find = [&](int x) { while (uf[x] != x) { uf[x] = uf[uf[x]]; x = uf[x]; } return x; };
     int ncon = sv[SV_NCON];
     for (int con = 0; con < ncon; ++con) {
       if (c.N(c.L().caddr)[con] < 0) continue;
       int t1 = c.bi(c.gi(c.N(c.L().cgeom)[2 * con], G_BODY), B_TREE);
       int t2 = c.bi(c.gi(c.N(c.L().cgeom)[2 * con + 1], G_BODY), B_TREE);
-      if (t1 >= 0) touched[t1] = 1;
-      if (t2 >= 0) touched[t2] = 1;
       if (t1 >= 0 && t2 >= 0) {
         int a = find(t1), b = find(t2);
         if (a != b) uf[a > b ? a : b] = a < b ? a : b;
@@ -3013,13 +2987,11 @@ __device__ void islands(const Ctx& c) {
     int nisl = 0;
     for (int t = 0; t < nt; ++t) {
       int r = find(t);
-      tisl[t] = !touched[t] ? -1 : (r == t ? nisl++ : tisl[r]);
+      tisl[t] = r == t ? nisl++ : tisl[r];
     }
     for (int i = 0; i < nisl; ++i) isz[i] = 0;
     for (int t = 0; t < nt; ++t) {
       int I = tisl[t];
-      toff[t] = 0;
-      if (I < 0) continue;
       toff[t] = isz[I];
       isz[I] += c.ti(t, T_DOFNUM);
     }
@@ -3039,7 +3011,7 @@ __device__ void islands(const Ctx& c) {
     int t = c.di(d, D_TREE), I = tisl[t], li = toff[t] + d - c.ti(t, T_DOFADR);
     c.N(c.L().disl)[d] = I;
     c.N(c.L().dloc)[d] = li;
-    if (I >= 0) c.N(c.L().idof)[istart[I] + li] = d;
+    c.N(c.L().idof)[istart[I] + li] = d;
   }
   sync();
 #endif
@@ -3176,41 +3148,6 @@ __device__ __forceinline__ bool flip_bit(const int* sv, int r) {
   return !sv[SV_FLIPOK] || (r < kFlipRows && ((flip_word(sv, r >> 6) >> (r & 63)) & 1ull));
 }
 
-// A lane's dof and its island (island, local index, size, first island-order slot, block
-// address), fixed within a substep: read once per solve when every dof has its own lane.  Size 0:
-// the dof's tree has no row.
-struct DofIsl { int I, li, n, st, blk; };
-
-__device__ __forceinline__ DofIsl dof_island(const Ctx& c, int d) {
-  DofIsl x{0, 0, 0, 0, 0};
-  if (d < c.m().nv) {
-    x.I = c.N(c.L().disl)[d];
-    if (x.I < 0) return x;
-    x.li = c.N(c.L().dloc)[d];
-    x.n = c.N(c.L().isz)[x.I];
-    x.st = c.N(c.L().istart)[x.I];
-    x.blk = c.N(c.L().iblk)[x.I];
-  }
-  return x;
-}
-
-// The trees without a row, of all dofs together.  Their part of a Newton step is the way to
-// qacc_smooth, and a step of length alpha leaves 1 - alpha of the distance e = qacc - qacc_smooth: the
-// iterates of the joint solve are those of its other dofs and rho, the product of the 1 - alpha, and
-// these trees enter its step lengths and stopping tests through three sums taken once.  So the blocks
-// hold no entries for them and no pass visits them (C3's arm: 45 of 171 entries, and pivots 6 instead
-// of 9; C5's parked objects: 21 entries each).  Control step before and after, same box: C3 x4096
-// 8.19 -> 7.78, C5 x16384 51.6 -> 48.5, C3 x67 4.00 -> 3.75 ms.
-struct FreeTrees {
-  real ss, gg, sg;   // e.e, (M e).(M e), e.(M e)
-  real rho;
-};
-
-// Whether dof i, one of this lane's (lane, lane + 64, ...), is in an island.
-__device__ __forceinline__ bool dof_on(const Ctx& c, const DofIsl& own, int i) {
-  return i < kLanes ? own.n > 0 : c.N(c.L().disl)[i] >= 0;
-}
-
 // Row forces/states (constraint_gradient, mjwarp_constraint.cu:107-201), qfrc_constraint = J^T f
 // and grad = Ma - qfrc_smooth - qfrc_constraint; returns ||grad||^2 (uniform).
 // *hchanged (when given): whether any row changed state (or is in the cone state, whose curvature
@@ -3218,7 +3155,7 @@ __device__ __forceinline__ bool dof_on(const Ctx& c, const DofIsl& own, int i) {
 // flips: record the rows whose state entered or left QUADRATIC, the only state property a
 // pyramidal-cone Hessian depends on (flip_word / flip_bit read them after the call).
 template <class V>
-__device__ real gradient(const Ctx& c, const V& v, const DofIsl& own, bool* hchanged = nullptr, bool flips = false) {
+__device__ real gradient(const Ctx& c, const V& v, bool* hchanged = nullptr, bool flips = false) {
   KModel& m = c.m();
   const int ncon = c.SV()[SV_NCON], nefc = c.SV()[SV_NEFC], K = m.maxpairdof;
   const int nfr = c.SV()[SV_NF];
@@ -3314,7 +3251,7 @@ __device__ real gradient(const Ctx& c, const V& v, const DofIsl& own, bool* hcha
   real g2 = 0.f;
   for (int i = c.lane(); i < m.nv; i += kLanes) {
     real q = qcon[i];
-    real g = dof_on(c, own, i) ? c.F(c.L().Ma)[i] - c.F(c.L().smooth)[i] - q : 0.f;
+    real g = c.F(c.L().Ma)[i] - c.F(c.L().smooth)[i] - q;
     c.F(c.L().qcon)[i] = q;                       // qfrc_constraint in the working set
     c.F(c.L().grad)[i] = g;
     g2 += g * g;
@@ -3555,7 +3492,6 @@ __device__ void hessian_inverse(const Ctx& c, const V& v, bool incremental = fal
     int cd = ent[2 * e], i = (cd >> 16) & 63, j = (cd >> 22) & 63;
     if (j > i) continue;
     int di = ent[2 * e + 1], dj = di - i + j;
-    if (disl[di] < 0) continue;
     *hent(H, iblk, disl[di], dloc[di], dloc[dj]) = (double)c.F(c.L().M)[e];
   }
 #endif
@@ -3620,7 +3556,7 @@ __device__ void hessian_inverse(const Ctx& c, const V& v, bool incremental = fal
 #ifndef MX_SLAB
 #pragma unroll
   for (int q = 0; q < kOwn; ++q) own[q] = hdecode(iblk, nisl, c.lane() + kLanes * q, total);
-  if (c.lane() < m.nv && disl[c.lane()] >= 0) {
+  if (c.lane() < m.nv) {
     int I = disl[c.lane()];
     sn_li = dloc[c.lane()]; sn_n = isz[I]; sn_col = istart[I] + sn_li; sn_blk = iblk[I];
   }
@@ -3641,7 +3577,7 @@ __device__ void hessian_inverse(const Ctx& c, const V& v, bool incremental = fal
     } 
     for (int d = c.lane() + kLanes; d < m.nv; d += kLanes) {
       int I = disl[d], li = dloc[d];
-      if (I >= 0 && k < isz[I]) {
+      if (k < isz[I]) {
         double hv = li >= k ? *hent(H, iblk, I, li, k) : *hent(H, iblk, I, k, li);
         col[istart[I] + li] = li == k ? 1.0 / hv : hv;
       }
@@ -3758,6 +3694,22 @@ __device__ __noinline__ bool hessian_rank1(const Ctx& c, const V& v) {
   return true;
 }
 
+// A lane's dof and its island (island, local index, size, first island-order slot, block
+// address), fixed within a substep: read once per solve when every dof has its own lane.
+struct DofIsl { int I, li, n, st, blk; };
+
+__device__ __forceinline__ DofIsl dof_island(const Ctx& c, int d) {
+  DofIsl x{0, 0, 0, 0, 0};
+  if (d < c.m().nv) {
+    x.I = c.N(c.L().disl)[d];
+    x.li = c.N(c.L().dloc)[d];
+    x.n = c.N(c.L().isz)[x.I];
+    x.st = c.N(c.L().istart)[x.I];
+    x.blk = c.N(c.L().iblk)[x.I];
+  }
+  return x;
+}
+
 // search = -H^-1 grad (the swept blocks hold -H^-1); returns search.search and grad.H^-1.grad.
 // own: the lane's dof island (every dof has its own lane)
 template <class V>
@@ -3776,10 +3728,10 @@ __device__ void direction(const Ctx& c, const V& v, const DofIsl& own, real& sea
     const int d = c.lane();
     real gd = d < m.nv ? grad[d] : 0.f;
     if constexpr (V::kStage) {   // the gradient in island order, in the window
-      if (own.n > 0) v.xs[own.st + own.li] = gd;
+      if (d < m.nv) v.xs[own.st + own.li] = gd;
       sync();
     }
-    if (own.n > 0) {
+    if (d < m.nv) {
       const int li = own.li, n = own.n;
       const auto* Hb = H + own.blk;
       const int* dl = idof + own.st;
@@ -3800,12 +3752,10 @@ __device__ void direction(const Ctx& c, const V& v, const DofIsl& own, real& sea
     return;
   }
   if constexpr (V::kStage) {   // the gradient in island order, in the window
-    for (int d = c.lane(); d < m.nv; d += kLanes)
-      if (disl[d] >= 0) v.xs[istart[disl[d]] + dloc[d]] = grad[d];
+    for (int d = c.lane(); d < m.nv; d += kLanes) v.xs[istart[disl[d]] + dloc[d]] = grad[d];
     sync();
   }
   for (int d = c.lane(); d < m.nv; d += kLanes) {
-    if (disl[d] < 0) continue;
     int I = disl[d], li = dloc[d], n = isz[I];
     const int* dl = idof + istart[I];
     double acc = 0.0;
@@ -3960,16 +3910,14 @@ constexpr int kRowsPerLane = 8;
 #endif
 
 template <class V>
-__device__ real linesearch(const Ctx& c, const V& v, const DofIsl& own, real search_dot, real free_sg, real& improvement,
-                           bool& converged) {
+__device__ real linesearch(const Ctx& c, const V& v, real search_dot, real& improvement, bool& converged) {
   KModel& m = c.m();
   const int nv = m.nv, nefc = c.SV()[SV_NEFC], ncon = c.SV()[SV_NCON];
   const real kNoise = 8.f * 1.1920929e-7f;
   const real* search = c.F(c.L().search);
   real* Mv = c.F(c.L().Mv);
   // Mv = M search, Jv = J search
-  for (int i = c.lane(); i < nv; i += kLanes)
-    if (dof_on(c, own, i)) Mv[i] = block_row_dot(c, c.F(c.L().M), search, i);
+  for (int i = c.lane(); i < nv; i += kLanes) Mv[i] = block_row_dot(c, c.F(c.L().M), search, i);
   rows_dot(c, v, search, v.rjv);
   if (m.opt_cone == 1) {
     const real ratio = 1.f / r_sqrt(m.opt_impratio);
@@ -4002,12 +3950,11 @@ __device__ real linesearch(const Ctx& c, const V& v, const DofIsl& own, real sea
   const real gtol = r_max(m.opt_tolerance * m.opt_ls_tolerance * r_sqrt(search_dot) * scale, 1e-6f);
   real g1 = 0.f, g2 = 0.f;
   for (int i = c.lane(); i < nv; i += kLanes) {
-    if (!dof_on(c, own, i)) continue;
     g1 += search[i] * (c.F(c.L().Ma)[i] - c.F(c.L().smooth)[i]);
     g2 += 0.5f * search[i] * Mv[i];
   }
-  g1 = wave_sum(g1) - free_sg;        // the trees without a row: search = -e
-  g2 = wave_sum(g2) + 0.5f * free_sg;
+  g1 = wave_sum(g1);
+  g2 = wave_sum(g2);
   LRow rows[kRowsPerLane];
 #pragma unroll
   for (int q = 0; q < kRowsPerLane; ++q) rows[q] = load_lrow(c, v, c.lane() + kLanes * q);
@@ -4080,7 +4027,6 @@ __device__ real linesearch(const Ctx& c, const V& v, const DofIsl& own, real sea
     }
   }
   for (int i = c.lane(); i < nv; i += kLanes) {
-    if (!dof_on(c, own, i)) continue;
     c.F(c.L().qacc)[i] += alpha * search[i];
     c.F(c.L().Ma)[i] += alpha * Mv[i];
   }
@@ -4099,26 +4045,13 @@ __device__ void newton_solve(const Ctx& c, const V& v) {
 #ifdef MX_SLAB
   hessian_maps(c, v);
 #endif
-  const DofIsl own = dof_island(c, c.lane());
-  FreeTrees ft{0.f, 0.f, 0.f, 1.f};
-  for (int i = c.lane(); i < nv; i += kLanes) {
-    const real ma = block_row_dot(c, c.F(c.L().M), qacc, i);
-    c.F(c.L().Ma)[i] = ma;
-    if (dof_on(c, own, i)) continue;
-    const real e = qacc[i] - c.F(c.L().qacc_smooth)[i], g = ma - c.F(c.L().smooth)[i];
-    c.F(c.L().search)[i] = e;   // kept for the end: no pass writes these dofs' search
-    ft.ss += e * e;
-    ft.gg += g * g;
-    ft.sg += e * g;
-  }
-  ft.ss = wave_sum(ft.ss);
-  ft.gg = wave_sum(ft.gg);
-  ft.sg = wave_sum(ft.sg);
+  for (int i = c.lane(); i < nv; i += kLanes) c.F(c.L().Ma)[i] = block_row_dot(c, c.F(c.L().M), qacc, i);
   rows_dot(c, v, qacc, v.rjaref);
   for (int r = c.lane(); r < nefc; r += kLanes) v.rjaref[r] -= v.raref[r];
   sync();
   real search_dot, decrement;
-  gradient(c, v, own);
+  const DofIsl own = dof_island(c, c.lane());
+  gradient(c, v);
   hessian_inverse(c, v);
   direction(c, v, own, search_dot, decrement);
   const real scale = m.meaninertia * nv, tol = m.opt_tolerance;
@@ -4127,14 +4060,12 @@ __device__ void newton_solve(const Ctx& c, const V& v) {
   while (m.opt_iterations > 0) {
     real improvement;
     bool ls_ok;
-    const real rho2 = ft.rho * ft.rho;
-    real alpha = linesearch(c, v, own, search_dot + rho2 * ft.ss, rho2 * ft.sg, improvement, ls_ok);
-    ft.rho *= 1.f - alpha;
+    real alpha = linesearch(c, v, search_dot, improvement, ls_ok);
     if (!ls_ok) ovf |= MX_OVERFLOW_LS_ITERATIONS;
     // the Hessian depends on the rows' states only (and on jaref for cone rows): when none changed,
     // the previous blocks still hold -H^-1
     bool hchanged;
-    const real grad_dot = gradient(c, v, own, &hchanged, true) + ft.rho * ft.rho * ft.gg;
+    real grad_dot = gradient(c, v, &hchanged, true);
     const bool fok = sv[SV_FLIPOK] != 0;
     unsigned long long fany = 0ull;
     int fcount = 0;
@@ -4158,7 +4089,6 @@ __device__ void newton_solve(const Ctx& c, const V& v) {
       }
     }
     direction(c, v, own, search_dot, decrement);
-    decrement += ft.rho * ft.rho * ft.sg;
     ++niter;
     real imp = improvement / scale, g = r_sqrt(grad_dot) / scale, mi = 0.5f * decrement / scale;
     bool done = alpha == 0.f || (imp > 0.f && imp < tol) || g < tol || mi < tol;
@@ -4167,8 +4097,6 @@ __device__ void newton_solve(const Ctx& c, const V& v) {
       break;
     }
   }
-  for (int i = c.lane(); i < nv; i += kLanes)
-    if (!dof_on(c, own, i)) qacc[i] = c.F(c.L().qacc_smooth)[i] + ft.rho * c.F(c.L().search)[i];
   if (v.copied)   // the rows' forces and states back to the working set (published, post-constraint)
     for (int r = c.lane(); r < nefc; r += kLanes) {
       c.F(c.L().rforce)[r] = v.rforce[r];

@@ -1,7 +1,7 @@
-"""Trees without a constraint row stay out of the Newton blocks; their part of the joint solve's steps
-is followed by three sums and the product of 1 - alpha.  The oracle solves all trees together: every
-tree's accelerations and the iteration counts of most worlds must be its (the parity bar 1e-4), and
-the free trees end within it of qacc_smooth.
+"""Trees without a constraint row (free trees) in the Newton solve, which solves all trees together as
+the oracle does: every tree's accelerations and the iteration counts of most worlds must be the
+oracle's (the parity bar 1e-4), the free trees end within it of qacc_smooth, take part in the iterates
+of a solve stopped early, and keep the precision of the solve's FP64 inverse.
 
 The arm free, held by a joint limit, or with dof friction rows; parked objects; both routes.
 """
@@ -10,9 +10,21 @@ import pytest
 
 from helpers import rel_err
 from libero_hip import native, scene as S
+from libero_hip.model import Model
 from test_gpu_contact_parity import _settled
 
 pytestmark = pytest.mark.gpu
+
+
+def _free_dofs(a, ncon, geoms, nefc, types, ids):
+    """The dofs of the trees that no contact and no joint or dof row of the world touches."""
+    touched = set()
+    for g in geoms[:2 * ncon]:
+        touched.add(int(a['body_treeid'][a['geom_body'][g]]))
+    for kind, row in zip(types[:nefc], ids[:nefc]):
+        if kind < 5:
+            touched.add(int(a['dof_treeid'][row if kind == 1 else a['jnt_dofadr'][row]]))
+    return np.array([int(t) not in touched for t in a['dof_treeid']])
 
 
 @pytest.mark.parametrize('config,arm', [('c1', 'free'), ('c3', 'free'), ('c3', 'limit'), ('c3', 'friction'),
@@ -36,23 +48,98 @@ def test_free_trees_follow_the_joint_solve(gpu_available, config, arm, route):
     torch.cuda.synchronize()
     g = {k: dd[k].cpu().numpy() for k in ('qacc', 'qacc_smooth', 'ncon', 'nefc', 'contact_geom', 'efc_type', 'efc_id')}
     a = {k: np.asarray(v).reshape(-1) for k, v in m.arrays.items()}
-    free = 0
+    free = arms = 0
     for w in range(nworld):
-        touched = set()
-        for c in range(g['ncon'][w, 0]):
-            for q in (0, 1):
-                touched.add(int(a['body_treeid'][a['geom_body'][g['contact_geom'][w, 2 * c + q]]]))
-        for r in range(g['nefc'][w, 0]):
-            kind, row = g['efc_type'][w, r], g['efc_id'][w, r]
-            if kind < 5:
-                touched.add(int(a['dof_treeid'][row if kind == 1 else a['jnt_dofadr'][row]]))
-        off = np.array([int(t) not in touched for t in a['dof_treeid']])
+        off = _free_dofs(a, g['ncon'][w, 0], g['contact_geom'][w], g['nefc'][w, 0], g['efc_type'][w], g['efc_id'][w])
         free += off.sum()
+        arms += off[0]
         if g['nefc'][w, 0]:
             scale = np.abs(od['qacc'][w]).max()
             assert np.abs(g['qacc'][w, off] - g['qacc_smooth'][w, off]).max(initial=0.0) < 1e-4 * scale
             assert np.abs(g['qacc'][w, off] - od['qacc'][w, off]).max(initial=0.0) < 1e-5 * scale
-    assert (free > 0) if arm == 'free' else free < nworld * 9 or config == 'c5'
+    assert free > 0 or arm == 'friction'
+    assert arms == (nworld if arm == 'free' else 0) or (arm == 'limit' and 0 < arms < nworld)
     assert rel_err(g['qacc'], od['qacc']) < 1e-4
     niter = dd['solver_niter'].cpu().numpy()[:, 0]
-    assert (niter == od['solver_niter'].reshape(-1)).mean() > 0.5
+    assert (niter == od['solver_niter'].reshape(-1)).mean() > 0.9     # measured: all of them
+
+
+@pytest.mark.parametrize('config,iterations', [('c3', 1), ('c3', 2), ('c5', 2)])
+@pytest.mark.parametrize('route', ['workspace', 'lds'])
+def test_free_trees_at_an_early_stop(gpu_available, config, iterations, route):
+    """Started from random accelerations and stopped after one or two steps, part of a free tree's
+    distance e from qacc_smooth is left in some worlds (the product of 1 - alpha, where alpha is not
+    1).  Both solvers leave the same there: measured 2e-6 to 7e-2 of what is left, by line searches
+    that stop a little apart, the medians below 1e-3 (bar 1e-2); free trees solved by themselves would
+    leave nothing, an error of all of it."""
+    import torch
+    nworld = 32
+    sc = S.make_scene(config, nworld, seed=6)
+    sc.options.iterations = iterations
+    m, dd, od, _ = _settled(config, nworld, settle=2, seed=6, scene=sc, workspace=None if route == 'workspace' else False)
+    rng = np.random.default_rng(60)
+    od.forward(None, native.FLAG_NO_CONTROL)
+    off = rng.uniform(-40, 40, (nworld, m.nv)) * (1 + np.arange(nworld))[:, None] / nworld
+    warm = (od['qacc'] + off).astype(np.float32)
+    dd['qacc_warmstart'].copy_(torch.from_numpy(warm))
+    od['qacc_warmstart'][:] = warm
+    dd.forward(None, native.FLAG_NO_CONTROL)
+    od.forward(None, native.FLAG_NO_CONTROL)
+    torch.cuda.synchronize()
+    g = {k: dd[k].cpu().numpy() for k in ('qacc', 'qacc_smooth', 'ncon', 'nefc', 'contact_geom', 'efc_type', 'efc_id')}
+    a = {k: np.asarray(v).reshape(-1) for k, v in m.arrays.items()}
+    left, err = [], []
+    for w in range(nworld):
+        if not g['nefc'][w, 0]:
+            continue
+        free = _free_dofs(a, g['ncon'][w, 0], g['contact_geom'][w], g['nefc'][w, 0], g['efc_type'][w], g['efc_id'][w])
+        if free.any():
+            e = np.abs(warm[w, free] - od['qacc_smooth'][w, free]).max()
+            left.append(np.abs(od['qacc'][w, free] - od['qacc_smooth'][w, free]).max() / e)
+            err.append(np.abs(g['qacc'][w, free] - od['qacc'][w, free]).max() / e)
+    left, err = np.array(left), np.array(err)
+    far = left > 1e-2
+    print('case', config, iterations, route, 'left', left[far], 'error', err[far], flush=True)
+    assert far.any() and np.median(err[far] / left[far]) < 1e-2
+
+
+@pytest.mark.parametrize('joints', ['plain', 'bare'])
+@pytest.mark.parametrize('route', ['workspace', 'lds'])
+def test_free_arm_keeps_the_solve_precision(gpu_available, joints, route):
+    """The free arm's acceleration against M x = qfrc_smooth solved in 64 bits on the published M and
+    qfrc_smooth, largest error over largest entry, median over the worlds.  The solve's last step
+    corrects qacc by an FP64 inverse, and half an ulp of the result is up to 6e-8; measured 1.02e-7 to
+    1.16e-7.  The FP32 inverse alone (qacc_smooth without that correction) measures 1.25e-7 to
+    1.33e-7.  bare: without damping and armature, so that qacc is integrated as it is."""
+    import torch
+    n = 512
+    sc = S.make_scene('c3', n, seed=8)
+    rng = np.random.default_rng(8)
+    if joints == 'bare':
+        for b in sc.bodies:
+            for j in b.joints:
+                j.damping = j.armature = 0.0
+    for k in range((sc.init_qpos.shape[1] - 9) // 7):      # every second object in the air
+        sc.init_qpos[:, 11 + 7 * k] += 0.25 if k % 2 else -0.0051
+    sc.init_qpos[:, :7] += rng.uniform(-0.4, 0.4, (n, 7))
+    sc.init_qvel[:, :7] = rng.uniform(-1, 1, (n, 7))
+    m = Model(sc)
+    d = native.DeviceData(native.DeviceModel(m), n, workspace=None if route == 'workspace' else False)
+    d['qpos'].copy_(torch.from_numpy(sc.init_qpos))
+    d['qvel'].copy_(torch.from_numpy(sc.init_qvel))
+    d['ctrl'][:, :7].copy_(torch.from_numpy(rng.uniform(-20, 20, (n, 7))))
+    d['body_active'].fill_(1)
+    d.forward(None, native.FLAG_BOOTSTRAP | native.FLAG_NO_CONTROL)
+    torch.cuda.synchronize()
+    g = {k: d[k].double().cpu().numpy() for k in ('qacc', 'qfrc_smooth', 'qfrc_constraint', 'M', 'nefc')}
+    assert (g['nefc'] > 0).all()
+    a = {k: np.asarray(v).reshape(-1) for k, v in m.arrays.items()}
+    nn, at = int(a['tree_dofnum'][0]), int(a['tree_madr'][0])
+    err = []
+    for w in range(n):
+        if not np.any(g['qfrc_constraint'][w, :nn]):
+            M = np.tril(g['M'][w, at:at + nn * nn].reshape(nn, nn))
+            x = np.linalg.solve(M + np.tril(M, -1).T, g['qfrc_smooth'][w, :nn])
+            err.append(np.abs(g['qacc'][w, :nn] - x).max() / np.abs(x).max())
+    print('case', joints, route, len(err), 'median error', np.median(err), flush=True)
+    assert len(err) > n // 2 and np.median(err) < 1.2e-7
