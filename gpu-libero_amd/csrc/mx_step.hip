@@ -129,9 +129,9 @@ inline void place_epa_region(Layout& L, const MxModel& m) {
 // either way, all the batch's worlds being resident at once).  What that buys is chosen so that a
 // world's results do not depend on the batch around it: row-group EPA and the contact staging, which
 // compute the same values as their fallbacks, and (waves > 1) the blocks of the wide kernel's further
-// waves; the Newton solve, whose Hessian rebuilds round differently when they run from a saved
-// assembly, keeps the layout of the small window (nwin).  (Row-group EPA instead of
-// one pair at a time: the LIBERO bowl-and-plate scene at 500 worlds 17.8 -> 15.1 ms per control step.)
+// waves; the Newton solve, whose arrays' place decides how it rounds, keeps the layout of the small
+// window (nwin).  (Row-group EPA instead of one pair at a time: the LIBERO bowl-and-plate scene at 500
+// worlds 17.8 -> 15.1 ms per control step.)
 // Returns whether the layout for so many waves fits the share.
 constexpr int kLdsGranule = 1280;   // bytes: LDS is allocated in such units
 constexpr int kWideScalars = 16;    // wide kernel: words after the scalar slots (counts per wave)
@@ -223,19 +223,12 @@ Layout make_layout(const MxModel& m) {
     L.win = kWindowWords;
     if (rows && (m.nmesh > 0 || !m.boxbox_primitive)) {
       int it = m.epa_iterations > 0 ? m.epa_iterations : 0;
-      // five vertices at most to start with and one more per expansion step.  (At the reference's
-      // 10 + 2 it vertices the dense-clutter scene's window took 2792 words and a CU held fifteen
-      // worlds; at 2480 it holds sixteen, and 8192 worlds are two full rounds instead of two and an
-      // almost empty third.)
-      L.epa_vc = 6 + it;
+      L.epa_vc = 6 + it;                // five vertices at most to start with and one more per expansion step
       L.epa_fc = 6 + 5 * it;
-      int poly = round_up(cvx::poly_words(L.epa_vc, L.epa_fc), 4), need = poly + kEpaRequest + cvx::kManifoldWords;
 #ifdef MX_SLAB
-      L.epa = 0;                        // at the start of the LDS window
-      L.epa_req = poly;
-      L.win = need > L.win ? round_up(need, 4) : L.win;
-      L.gpose = need;
+      L.epa = 0;                        // at the start of the LDS window, which is sized below
 #else
+      int poly = round_up(cvx::poly_words(L.epa_vc, L.epa_fc), 4), need = poly + kEpaRequest + cvx::kManifoldWords;
       // in reals: the polytope, the request block and the manifold's clip block
       L.epa = need * kRealWords <= L.tisl - L.rid ? L.rid : take(need * kRealWords);
       L.epa_req = L.epa + poly * kRealWords;
@@ -277,11 +270,32 @@ Layout make_layout(const MxModel& m) {
   // the islands' tables (islands(): 7 ntree + 2 words, two per contact and two per dof)
   if (m.njmax > 0 && L.win < 7 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv)
     L.win = round_up(7 * m.ntree + 2 + 2 * m.nconmax + 2 * m.nv, 4);
-  // the geoms' collision records after the EPA block
-  if (m.njmax > 0 && L.win < L.gpose + GP_WORDS * m.ngeom) L.win = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
-  // then the hull vertices (4 words each), read by every support-point search of the stage
-  L.meshw = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
-  if (m.njmax > 0 && m.nmeshvert > 0 && L.win < L.meshw + 4 * m.nmeshvert) L.win = round_up(L.meshw + 4 * m.nmeshvert, 4);
+  // the collision stage: the EPA polytope with its request and clip blocks, the geoms' collision
+  // records, then the hull vertices (4 words each), read by every support-point search of the stage
+  if (m.njmax > 0) {
+    const int others = L.win, it = m.epa_iterations > 0 ? m.epa_iterations : 0;
+    auto place = [&](int vc) {
+      L.win = others;
+      if (L.epa == 0) {
+        L.epa_vc = vc;
+        L.epa_req = round_up(cvx::poly_words(L.epa_vc, L.epa_fc), 4);
+        L.gpose = L.epa_req + kEpaRequest + cvx::kManifoldWords;
+      }
+      L.meshw = round_up(L.gpose + GP_WORDS * m.ngeom, 4);
+      if (L.win < L.meshw + 4 * m.nmeshvert) L.win = round_up(L.meshw + 4 * m.nmeshvert, 4);
+    };
+    // The reference's 10 + 2 it vertices, or the 6 + it that an expansion can make where those let
+    // sixteen worlds share a CU and the former do not: the dense-clutter scene's window takes 2792 or
+    // 2480 words, fifteen or sixteen worlds per CU, so that its 8192 worlds are two full rounds and not
+    // two and an almost empty third (71.3 -> 59.1 ms per control step).  Elsewhere the window, which the Newton solve
+    // lays itself out in too, stays the larger: in a smaller one more worlds solve on the slab's
+    // arrays, at the same precision but rounded otherwise (the LIBERO scenes' results moved).
+    place(10 + 2 * it);
+    if (L.win > kWindowWords) {
+      place(6 + it);
+      if (L.win > kWindowWords) place(10 + 2 * it);
+    }
+  }
   L.gpose0 = L.gpose;
   place_epa_region(L, m);
   L.nwin = L.win;
