@@ -4522,7 +4522,7 @@ __device__ void store_world(const Ctx& c, int integrated) {
 // instantiation carries none of the collision / Newton code, so its register allocation is that
 // of the smooth stages alone.
 // Minimum waves per SIMD the register allocation must allow.  In LDS the contact kernel holds
-// 60-125 KB per world, so at most two worlds share a CU and registers are not the limit.  With the
+// 40-125 KB per world, so at most four worlds share a CU and registers are not the limit.  With the
 // working set in workspace slabs the only limit is registers: four waves per SIMD (128 VGPRs)
 // hides the slabs' memory latency best (measured 1 to 8 waves per SIMD: 4 is fastest on C3, C4,
 // C5; fewer registers spill more).
@@ -4590,7 +4590,6 @@ __device__ __forceinline__ void add_stats(const Ctx& c) {
   sv[SV_STAT + 3] += sv[SV_NITER] * sv[SV_NEFC];
 }
 
-#ifdef MX_SLAB
 template <bool kRows>
 // The parameter block is read through params() (the kernel argument segment), never through the
 // by-value parameter, so no private copy of it is made.
@@ -4620,6 +4619,7 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   if (!(m.opt_disableflags & (1 << 15)))
     for (int i = 0; i < m.nv; ++i) damped |= c.df(i, D_DAMP) > 0.f;
   int integrated = 0;
+#ifdef MX_SLAB
   // A launch lasts as long as its slowest world, and the worlds of one CU share its SIMDs: a world
   // whose substeps trail its group's mean by more than one and a half raises its wave's issue
   // priority until it catches up.  Each substep start adds one to the group's counter (a relaxed
@@ -4630,8 +4630,10 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   const unsigned int nw = (unsigned int)((p.d.nworld - (w & (kPaceGroups - 1)) + kPaceGroups - 1) / kPaceGroups);
   unsigned int* pace_ctr = g_substeps_started + (w & (kPaceGroups - 1)) * kPaceStride;
   const bool pace = kRows && p.pace;
+#endif
   for (int s = 0; s < substeps; ++s) {
     const int policy = (flags & MX_FLAG_POLICY_FIRST) && s == 0;
+#ifdef MX_SLAB
     if (pace) {
       // at this world's start of substep s - 1 the group's worlds had started before / nw
       // substeps on average, against this world's s - 1: behind by more than 1.5 substeps
@@ -4640,6 +4642,7 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
       else __builtin_amdgcn_s_setprio(0);
       if (threadIdx.x == 0) started = __hip_atomic_fetch_add(pace_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+#endif
     kinematics(c);
     com_pos(c);
     crb_mass(c);
@@ -4681,6 +4684,7 @@ __global__ __launch_bounds__(kLanes, kMinWaves(kRows)) void control_step_kernel(
   store_world(c, integrated);
 }
 
+#ifdef MX_SLAB
 // The same control step with kWaves wavefronts per world, for batches that leave wave slots free
 // (launch_kernel): there a substep is one wave's latency, and most of it is work that need not wait
 // for the rest.  All waves make the collision records and filter the pair table (a part each); then
@@ -4814,9 +4818,10 @@ __global__ __launch_bounds__(kWaves * kLanes, kMinWaves(true)) void control_step
 // The LDS route's control step of models with constraint rows, with two wavefronts per world: while
 // wave 0 collides, wave 1 runs the stages that need the positions only (com, mass matrix and
 // inverses, velocity, the FP64 controller, actuation); everything else is wave 0's.  A CU holds one
-// or two such worlds in its LDS, so the second wave's slot is free.  Between the workgroup barriers
+// or two worlds of the contact scenes in its LDS, so the second wave's slot is free.  Between the workgroup barriers
 // the waves write disjoint parts of the working set (the EPA polytope aliases the rows, which wave 1
-// does not touch).  (FP64 route, C3 x300: 12.1 -> 10.6 ms per control step.)
+// does not touch).  (FP64 route, C3 x300: 12.1 -> 10.6 ms per control step.)  Not for batches that would
+// fill more of a CU with one wave per world (two_waves()).
 __global__ __launch_bounds__(2 * kLanes, kMinWaves(true)) void control_step_kernel_rows2(Params) {
   {
     typedef const __attribute__((address_space(4))) unsigned char KByte;
@@ -4997,7 +5002,6 @@ __global__ __launch_bounds__(256) void image_kernel(Params) {
 }
 #endif
 
-#ifdef MX_SLAB
 // The current device's CU count (0 when it cannot be had), asked once per device.
 static int cu_count() {
   static int ncu[64];   // filled on first use (a benign race: every writer stores the same)
@@ -5011,11 +5015,27 @@ static int cu_count() {
   return ncu[dev];
 }
 
+#ifdef MX_SLAB
 // Whether a launch's worlds are all resident at once: each CU holds 4 waves per SIMD (the kernel's
 // register budget) or fewer when their LDS windows fill its 160 KB.
 static bool all_resident(int nworld, size_t shared, int ncu) {
   const long long by_lds = MX_LDS_BUDGET / (long long)shared, per_cu = by_lds < 4 * kMinWaves(true) ? by_lds : 4 * kMinWaves(true);
   return (long long)nworld <= (long long)ncu * per_cu;
+}
+#else
+// Whether a launch of a model with constraint rows takes two waves per world (rows2).  Either kernel's
+// registers leave a SIMD one wave, so a CU holds as many worlds as its LDS, up to four of one wave or
+// two of two: two waves wherever the batch then needs no more rounds of resident worlds.  Control step
+// with one and two waves, arm, table and one box at 24 contacts (40 KB, four worlds per CU): 512 worlds
+// 2.69 and 1.94 ms, 700 worlds 2.72 and 3.69, 8192 worlds 22.2 and 30.3; FP64, arm and table (51 KB,
+// three): 512 worlds 1.35 and 1.07, 8192 worlds 13.8 and 19.8.
+inline bool two_waves(int nworld, size_t shared, int ncu) {
+  const int by_lds = (int)(MX_LDS_BUDGET / shared);
+  auto rounds = [&](int most) {
+    const long long resident = (long long)(ncu > 0 ? ncu : 1) * (by_lds < most ? by_lds : most);
+    return (nworld + resident - 1) / resident;
+  };
+  return rounds(2) <= rounds(4);
 }
 #endif
 
@@ -5023,8 +5043,8 @@ int launch_kernel(const MxModel* m, const MxData* d, const int32_t* mask, int su
                   const MxObsPlan* obs) {
   MxObsPlan none{};
   Params p{*m, *d, make_layout(*m), image_layout(*m), substeps, flags, mask, obs ? *obs : none, 0};
-#ifdef MX_SLAB
   const int ncu = cu_count();
+#ifdef MX_SLAB
   // Waves per world: as many as keep every world resident in the CU's sixteen wave slots, four at
   // most.  Control step with one, two and four waves: C3 x67 5.17, 4.33, 4.00 ms; C1 x2 4.14, 3.34,
   // 3.29; the LIBERO bowl-and-plate scene x500 15.1, 14.2, 11.2; C3 x1024 (four worlds per CU) 6.21,
@@ -5053,7 +5073,9 @@ int launch_kernel(const MxModel* m, const MxData* d, const int32_t* mask, int su
   else
     hipLaunchKernelGGL(control_step_kernel<false>, dim3(d->nworld), dim3(kLanes), shared, (hipStream_t)stream, p);
 #else
-  if (m->njmax > 0)
+  if (m->njmax > 0 && !two_waves(d->nworld, shared, ncu))
+    hipLaunchKernelGGL(control_step_kernel<true>, dim3(d->nworld), dim3(kLanes), shared, (hipStream_t)stream, p);
+  else if (m->njmax > 0)
     hipLaunchKernelGGL(control_step_kernel_rows2, dim3(d->nworld), dim3(2 * kLanes), shared, (hipStream_t)stream, p);
   else
     hipLaunchKernelGGL(control_step_kernel_smooth, dim3(d->nworld), dim3(2 * kLanes), shared, (hipStream_t)stream, p);

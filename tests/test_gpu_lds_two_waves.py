@@ -1,6 +1,8 @@
 """The LDS route's two-wave kernel: the same worlds bit for bit at any place and size of a batch, on
 both precisions, and to FP32 rounding the workspace route's result (one substep: positions 1e-6,
-velocities and accelerations by their scale 1e-4, the parity bar of the two routes)."""
+velocities and accelerations by their scale 1e-4, the parity bar of the two routes).  Models small
+enough for three or four worlds in a CU's LDS take one wave per world in batches that fill them so:
+the same bits on either side."""
 import numpy as np
 import pytest
 
@@ -12,9 +14,10 @@ from libero_hip.model import Model
 pytestmark = pytest.mark.gpu
 
 
-def run(name, nworld, flags, substeps):
+def run(name, nworld, flags, substeps, nobjects=None, nconmax=64):
     import torch
-    sc = S.make_scene(name, 8, seed=4)
+    sc = S.make_scene(name, 8, seed=4, nobjects=nobjects)
+    sc.options.nconmax = nconmax
     for k in range((sc.init_qpos.shape[1] - 9) // 7):
         sc.init_qpos[:, 11 + 7 * k] -= 0.0051
     pick = np.arange(nworld) % 8
@@ -47,3 +50,22 @@ def test_two_waves(gpu_available, name, route):
     assert np.abs(a['qpos'] - b['qpos']).max() < 1e-6
     for k in ('qvel', 'qacc', 'M', 'qfrc_bias', 'osc_tau'):
         assert rel_err(a[k], b[k]) < 1e-4, k
+
+
+@pytest.mark.parametrize('route,nobjects', [('lds', 1), ('fp64', 0)])
+def test_one_wave_and_two_waves_agree(gpu_available, route, nobjects):
+    import torch
+    flags = native.FLAG_LDS if route == 'lds' else native.FLAG_FP64
+    sc = S.make_scene('c1', 1, nobjects=nobjects)
+    sc.options.nconmax = 24
+    dm = native.DeviceModel(Model(sc))
+    assert (dm.lds_bytes() if route == 'lds' else dm.lds_bytes_fp64()) <= 163840 // 3     # three worlds per CU at least
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    one = run('c1', 8, flags, 6, nobjects, 24)
+    assert one['nefc'].max() > 0 or nobjects == 0
+    for nworld in (2 * cus, 2 * cus + 1, 3 * cus, 6 * cus + 3):      # two waves; one wave
+        print('case', route, nworld, flush=True)
+        many = run('c1', nworld, flags, 6, nobjects, 24)
+        for k in FIELDS:
+            pick = np.arange(nworld) % 8
+            np.testing.assert_array_equal(many[k], one[k][pick], err_msg='%s %d' % (k, nworld))

@@ -5,6 +5,8 @@
   sixteen worlds share a CU;
 * a launch that widens it (more row-group EPA blocks, several waves per world) stays inside the CU's
   LDS, leaves the Newton solve its layout, and keeps the parts apart that waves write at once.
+
+And the LDS route's choice of one or two waves per world, which must not cost a batch residency.
 """
 import ctypes as ct
 import subprocess
@@ -30,21 +32,28 @@ extern "C" int window(const MxModel* m, int nworld, int ncu, int waves, int* out
 }
 extern "C" int polytope_words(int vertices, int faces) { return mx_slab::cvx::poly_words(vertices, faces); }
 '''
+WAVES_SOURCE = '''
+#include "%s"
+extern "C" int two_waves(int nworld, int bytes, int ncu) { return mx_f64::two_waves(nworld, bytes, ncu); }
+'''
 REQUEST, CLIP, SCALARS, COUNTS, CUS = 48, 88, 48, 16, 256
 SCENES = ['c1', 'c3', 'c4', 'c5', 'libero_spatial_bowl_plate', 'libero_goal_wine_rack']
 
 
+def compiled(at, source):
+    """The host half of a HIP source alone: an empty device image, nothing launched."""
+    import build
+    (at / 'source.hip').write_text(source)
+    subprocess.run([build.hipcc(), '--offload-arch=gfx950', '--offload-host-only', '-fuse-cuid=none', '-O0', '-std=c++17',
+                    '-fPIC', '-shared', '-o', str(at / 'source.so'), str(at / 'source.hip'),
+                    '-Wl,--defsym,__hip_fatbin=0'], check=True)
+    return ct.CDLL(str(at / 'source.so'))
+
+
 @pytest.fixture(scope='module')
 def lib(tmp_path_factory):
-    import build
-    at = tmp_path_factory.mktemp('window')
     slab = ROOT / 'gpu-libero_amd' / 'csrc' / 'mx_step_slab.hip'
-    (at / 'window.hip').write_text(SOURCE % (slab, ', '.join('L.' + n for n in NAMES), len(NAMES)))
-    # the host half only: nothing is registered with the runtime (an empty device image), nothing launched
-    subprocess.run([build.hipcc(), '--offload-arch=gfx950', '--offload-host-only', '-fuse-cuid=none', '-O0', '-std=c++17',
-                    '-fPIC', '-shared', '-o', str(at / 'window.so'), str(at / 'window.hip'),
-                    '-Wl,--defsym,__hip_fatbin=0'], check=True)
-    return ct.CDLL(str(at / 'window.so'))
+    return compiled(tmp_path_factory.mktemp('window'), SOURCE % (slab, ', '.join('L.' + n for n in NAMES), len(NAMES)))
 
 
 def model(name):
@@ -104,3 +113,15 @@ def test_widened_window(lib, name, waves):
                 assert w['ewords'] == w['gpose'] and w['swin'] >= w['ewin'] + (waves - 2) * w['ewords']
                 assert w['swin'] + smooth <= w['win'] and w['ewin'] % 4 == w['swin'] % 2 == 0
     assert taken > 0
+
+
+def test_lds_route_waves(tmp_path):
+    """Two waves per world exactly where one wave per world would take as many rounds of resident
+    worlds (a CU holds as many as its LDS, four of one wave or two of two)."""
+    lib = compiled(tmp_path, WAVES_SOURCE % (ROOT / 'gpu-libero_amd' / 'csrc' / 'mx_step_f64.hip'))
+    for nbytes in (20000, 40240, 48976, 50720, 58048, 69104, 85136, 163840):
+        fit = layout.LDS_BUDGET // nbytes
+        for nworld in (1, 16, CUS, CUS + 1, 2 * CUS, 2 * CUS + 1, 3 * CUS, 4 * CUS, 4 * CUS + 1, 8192, 16384):
+            rounds = lambda most: -(-nworld // (CUS * min(fit, most)))  # noqa: E731
+            assert bool(lib.two_waves(nworld, nbytes, CUS)) == (rounds(2) <= rounds(4)), (nbytes, nworld)
+            assert fit > 2 or lib.two_waves(nworld, nbytes, CUS)
