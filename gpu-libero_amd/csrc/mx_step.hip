@@ -80,8 +80,8 @@ constexpr int kStagePair = 18, kStageContact = 8;
 constexpr int kWindowWords = 2512;
 constexpr int kLdsScalars = 48;     // workspace route: the misc and sv slots, in LDS after the window
 // workspace route: per geom in the LDS window during the collision stage, first four words for the
-// broadphase (position and reach: bounding radius + margin + gap, negative for a plane, NaN on a
-// parked body; one 16-byte read), then for all geoms a record of the rest (rotation, size, type with
+// broadphase (position and reach: bounding radius + margin + gap where these are positive, -1 for a
+// plane, NaN on a parked body; one 16-byte read), then for all geoms a record of the rest (rotation, size, type with
 // the hull's vertex count above its eight bits, margin, gap, bounding radius, hull vertices' image
 // word offset; an odd stride, so lanes reading consecutive records meet no bank twice)
 enum : int { GP_MAT = 0, GP_SIZE = 9, GP_TYPE = 12, GP_MARGIN = 13, GP_GAP = 14, GP_RBOUND = 15, GP_VERT = 16,
@@ -2294,7 +2294,8 @@ __device__ __noinline__ bool convex_epa_rows(const Ctx& c, ConvexLane& __restric
 // candidates ends with its ballot.  (One round at a time, on six to thirteen 4-byte reads in
 // branches, the LIBERO bowl-and-plate scene's 13843 pairs took 98 us of a 757 us substep.)  Out of
 // line: inlined, its registers pushed the kernel body's values to scratch.  The bound is rounded up
-// past the sums' rounding, so no pair is lost that the narrowphase's own thresholds would accept.
+// past the sums' rounding and takes a negative margin or gap as zero (a pair's threshold is the sum of
+// its geoms' or the larger), so no pair is lost that the narrowphase's own thresholds would accept.
 constexpr int kPairBatch = 4;
 
 __device__ __noinline__ int broadphase(const Ctx& c, int first, int last) {
@@ -2325,7 +2326,7 @@ __device__ __noinline__ int broadphase(const Ctx& c, int first, int last) {
       keep[u] = dx * dx + dy * dy + dz * dz <= bound * bound && !plane;
       if (__ballot(plane)) {   // plane against a geom's bounding sphere
         const sfloat* gm1 = c.gmat(g1[u]);
-        const real thr = b[u].w + c.gmargin(g1[u]) + c.ggap(g1[u]);
+        const real thr = b[u].w + r_max(c.gmargin(g1[u]), 0.f) + r_max(c.ggap(g1[u]), 0.f);
         if (plane) {
           const real h = gm1[2] * dx + gm1[5] * dy + gm1[8] * dz;
           keep[u] = h - thr <= 4e-6f * (r_abs(h) + r_abs(thr));
@@ -2369,7 +2370,7 @@ __device__ __forceinline__ void collision_records(const Ctx& c, int tid, int n) 
       nvert = rec[1];
     }
     for (int k = 0; k < 3; ++k) bp[GP_BROAD * g + k] = pos[k];
-    bp[GP_BROAD * g + 3] = parked ? __builtin_nanf("") : (type == GT_PLANE ? -1.f : rbound + margin + gap);
+    bp[GP_BROAD * g + 3] = parked ? __builtin_nanf("") : (type == GT_PLANE ? -1.f : rbound + r_max(margin, 0.f) + r_max(gap, 0.f));
     sfloat* r = gp + GP_RECORD * g;
     for (int k = 0; k < GP_TYPE; ++k) r[k] = x[k];
     ((sint*)r)[GP_TYPE] = type | (nvert << 8);

@@ -16,7 +16,7 @@ from libero_hip.model import Model
 pytestmark = pytest.mark.gpu
 
 
-def cluster_scene(nbody, per_body, nworld, seed, mpr, parked):
+def cluster_scene(nbody, per_body, nworld, seed, mpr, parked, margins=(0.0, 0.002), gaps=(0.0, 0.001)):
     rng = np.random.default_rng(seed)
     arm, actuators, osc, q_ready = S._arm()
     bodies = [S._world(table=False)] + arm
@@ -26,7 +26,7 @@ def cluster_scene(nbody, per_body, nworld, seed, mpr, parked):
         for _ in range(per_body):
             b.geoms.append(S.Geom(S.SPHERE, size=(float(rng.uniform(0.005, 0.02)), 0.0, 0.0), condim=1,
                                   pos=tuple(float(x) for x in rng.uniform(-0.05, 0.05, 3)),
-                                  margin=float(rng.choice([0.0, 0.002])), gap=float(rng.choice([0.0, 0.001]))))
+                                  margin=float(rng.choice(margins)), gap=float(rng.choice(gaps))))
         bodies.append(b)
     opts = S.Options()
     opts.nconmax, opts.mpr = 256, mpr
@@ -49,8 +49,18 @@ def cluster_scene(nbody, per_body, nworld, seed, mpr, parked):
                          [(1, 1, False, False), (2, 3, False, True), (3, 4, True, False), (4, 5, False, True),
                           (5, 7, True, True)])
 def test_batched_filter_keeps_every_pair(gpu_available, nbody, per_body, mpr, parked):
+    compare(cluster_scene(nbody, per_body, 32, 10 * nbody + per_body, mpr, parked))
+
+
+@pytest.mark.parametrize('mpr', [False, True])
+def test_negative_margins_and_gaps(gpu_available, mpr):
+    """A margin below minus a sphere's radius, and a pair whose threshold is the larger of a negative
+    margin and zero: no pair is lost, and no sphere is taken for a plane."""
+    compare(cluster_scene(5, 6, 32, 77, mpr, False, margins=(-0.03, -0.004, 0.0, 0.002), gaps=(-0.002, 0.0, 0.001)))
+
+
+def compare(sc):
     import torch
-    sc = cluster_scene(nbody, per_body, 32, 10 * nbody + per_body, mpr, parked)
     m = Model(sc)
     om, od = make_oracle(m, sc.nworld, fp32_model=True)
     dd = native.DeviceData(native.DeviceModel(m), sc.nworld)
