@@ -5297,8 +5297,9 @@ __global__ __launch_bounds__(kLanes, 2) void osc_kernel(OscParams) {
 #pragma unroll
   for (int k = 0; k < 9; ++k) eer[k] = d.osc_ee_rot[9 * w + k];
   const double bias = d.osc_bias[on * w + jn];
-  const double pdj = 10.0 * (d.osc_q0[on * w + jn] - (double)d.osc_q[on * w + jn]) -
+  const double pdn = 10.0 * (d.osc_q0[on * w + jn] - (double)d.osc_q[on * w + jn]) -
                      6.324555320336759 * (double)d.osc_qvel[on * w + jn];
+  const double pdj = j < on ? pdn : 0.0;   // past the joints a zero of M meets it, which must not be infinite
   const double ev = d.osc_ee_vel[6 * w + j6], kpj = d.osc_gains[12 * w + j6], kdj = d.osc_gains[12 * w + 6 + j6];
 
   // M^-1

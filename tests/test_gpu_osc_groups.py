@@ -1,5 +1,6 @@
 """mx_osc packs eight worlds into a wavefront: batches around whole waves, with worlds in one wave that
-take different ways through the controller, each against the FP64 oracle on the same inputs."""
+take different ways through the controller, each against the FP64 oracle on the same inputs; and an
+infinite joint state, which must reach the torques as it does there."""
 import numpy as np
 import pytest
 
@@ -77,3 +78,42 @@ def test_osc_groups(gpu_available, joints, nworld, uncouple, policy):
         np.testing.assert_allclose(after['ctrl'][w, m.arrays['osc_actuator']], ctrl, rtol=1e-6, atol=1e-6)
         others = np.setdiff1d(np.arange(m.nu), m.arrays['osc_actuator'])
         assert np.array_equal(after['ctrl'][w, others], before['ctrl'][w, others])
+
+
+def test_infinite_joint_state(gpu_available):
+    """An infinite first joint velocity: the posture torques are infinite, and a torque is infinite or NaN
+    as its nullspace terms' signs agree or not.  With seven joints a wave's eighth lane holds no joint."""
+    import torch
+    from libero_hip import native, scene as S
+    from oracle import oracle as O
+    nworld = 200
+    m, dd, _ = _pair('c2', nworld, scene=S.make_scene('c2', nworld, seed=0))
+    n = m.osc_ndof
+    rng = np.random.default_rng(71)
+    L = rng.normal(size=(nworld, n, n)) * 0.2 + np.eye(n)
+    qvel = rng.normal(size=(nworld, n))
+    qvel[:, 0] = np.where(np.arange(nworld) % 2, np.inf, -np.inf)
+    fields = dict(osc_mass=(L @ L.transpose(0, 2, 1)).reshape(nworld, -1), osc_jac=rng.normal(size=(nworld, 6 * n)),
+                  osc_q=rng.normal(size=(nworld, n)), osc_qvel=qvel, osc_bias=rng.normal(size=(nworld, n)),
+                  osc_ee_pos=rng.normal(size=(nworld, 3)), osc_ee_rot=np.tile(np.eye(3).reshape(9), (nworld, 1)),
+                  osc_ee_vel=rng.normal(size=(nworld, 6)), osc_goal_pos=rng.normal(size=(nworld, 3)),
+                  osc_goal_rot=np.tile(np.eye(3).reshape(9), (nworld, 1)), osc_action=rng.uniform(-1, 1, (nworld, 7)))
+    for k, v in fields.items():
+        dd[k].copy_(torch.from_numpy(np.ascontiguousarray(v)).reshape(dd[k].shape))
+    inp = {k: _np(dd['osc_' + k]).reshape(nworld, -1) for k in ('mass', 'jac', 'q', 'qvel', 'bias', 'ee_pos', 'ee_rot', 'ee_vel')}
+    grip = _np(dd['osc_gripper']).copy()
+    dd.osc(0)
+    torch.cuda.synchronize()
+    tau, ctrl = _np(dd['osc_tau']).reshape(nworld, -1), _np(dd['ctrl']).reshape(nworld, -1)
+    acts = m.arrays['osc_actuator']
+    infinite = 0
+    for w in range(nworld):
+        _, want, wctrl, *_ = O.osc({k: v[w] for k, v in inp.items()}, fields['osc_action'][w], _np(dd['osc_gains'])[w],
+                                   _np(dd['osc_q0'])[w], m.arrays['actuator_ctrlrange'][acts].reshape(-1),
+                                   fields['osc_goal_pos'][w], fields['osc_goal_rot'][w], grip[w], policy=False,
+                                   uncouple=m.osc_uncouple, speed=float(np.float32(m.osc_gripper_speed)))
+        infinite += np.isinf(want).sum()
+        assert not np.isfinite(want).any()
+        np.testing.assert_array_equal(tau[w], want)
+        np.testing.assert_array_equal(ctrl[w, acts[:n]], wctrl[:n].astype(np.float32))
+    assert infinite > 20
