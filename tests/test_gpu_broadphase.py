@@ -1,8 +1,9 @@
 """The broadphase's batched filter of the pair table against the oracle's contacts.
 
-Sphere clusters on several free bodies give pair tables from below one round of 64 pairs to several
-batches with a remainder (the printed counts), with margins and gaps, under both margin rules, and
-with a parked body.  Sphere contacts are closed forms, so the contacts' geom pairs and order are those of the
+Sphere clusters on several free bodies give pair tables from below one round of 64 pairs (the counts
+are printed) to several batches of 256 with a remainder in each wave's part, with margins and gaps, under
+both margin rules, and with a parked body; a batch of more than eight worlds per CU runs the one-wave
+kernel, which filters the whole table in one call.  Sphere contacts are closed forms, so the contacts' geom pairs and order are those of the
 oracle exactly, and every pair within its threshold must be there: a pair the filter lost is missing.
 Positions agree to 1e-5 m (FP32 rounding of poses of order 1 m and of normals of centimetre offsets).
 """
@@ -47,9 +48,15 @@ def cluster_scene(nbody, per_body, nworld, seed, mpr, parked, margins=(0.0, 0.00
 
 @pytest.mark.parametrize('nbody,per_body,mpr,parked',
                          [(1, 1, False, False), (2, 3, False, True), (3, 4, True, False), (4, 5, False, True),
-                          (5, 7, True, True)])
+                          (5, 7, True, True), (7, 9, False, True), (7, 9, True, False)])
 def test_batched_filter_keeps_every_pair(gpu_available, nbody, per_body, mpr, parked):
     compare(cluster_scene(nbody, per_body, 32, 10 * nbody + per_body, mpr, parked))
+
+
+def test_whole_table_in_one_call(gpu_available):
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    compare(cluster_scene(7, 9, 32, 5, False, True), 8 * cus + 32)
 
 
 @pytest.mark.parametrize('mpr', [False, True])
@@ -59,21 +66,24 @@ def test_negative_margins_and_gaps(gpu_available, mpr):
     compare(cluster_scene(5, 6, 32, 77, mpr, False, margins=(-0.03, -0.004, 0.0, 0.002), gaps=(-0.002, 0.0, 0.001)))
 
 
-def compare(sc):
+def compare(sc, nworld=None):
+    """The scene's worlds, repeated to a batch of nworld, against the oracle."""
     import torch
     m = Model(sc)
     om, od = make_oracle(m, sc.nworld, fp32_model=True)
-    dd = native.DeviceData(native.DeviceModel(m), sc.nworld)
-    dd['qpos'].copy_(torch.from_numpy(sc.init_qpos))
-    od['qpos'][:] = dd['qpos'].double().cpu().numpy()
-    dd['body_active'].copy_(torch.from_numpy(od['body_active'].astype(np.int32)))
+    nworld = nworld or sc.nworld
+    pick = np.arange(nworld) % sc.nworld
+    dd = native.DeviceData(native.DeviceModel(m), nworld)
+    dd['qpos'].copy_(torch.from_numpy(sc.init_qpos[pick]))
+    od['qpos'][:] = dd['qpos'].double().cpu().numpy()[:sc.nworld]
+    dd['body_active'].copy_(torch.from_numpy(od['body_active'].astype(np.int32)[pick]))
     dd.forward(None, native.FLAG_BOOTSTRAP | native.FLAG_NO_CONTROL)
     od.forward(None, native.FLAG_BOOTSTRAP | native.FLAG_NO_CONTROL)
     torch.cuda.synchronize()
     ncon = dd['ncon'].cpu().numpy()[:, 0]
     print('pairs', m.arrays['pair_geom'].reshape(-1, 2).shape[0], 'contacts', ncon.sum(), flush=True)
-    assert ncon.max() < m.nconmax and np.array_equal(ncon, od['ncon'].reshape(-1))
+    assert ncon.max() < m.nconmax and np.array_equal(ncon, od['ncon'].reshape(-1)[pick])
     geom, pos = dd['contact_geom'].cpu().numpy(), dd['contact_pos'].double().cpu().numpy()
     for w, c in enumerate(ncon):
-        assert np.array_equal(geom[w, :2 * c], od['contact_geom'][w, :2 * c])
-        assert np.abs(pos[w, :3 * c] - od['contact_pos'][w, :3 * c]).max(initial=0.0) < 1e-5
+        assert np.array_equal(geom[w, :2 * c], od['contact_geom'][pick[w], :2 * c])
+        assert np.abs(pos[w, :3 * c] - od['contact_pos'][pick[w], :3 * c]).max(initial=0.0) < 1e-5
