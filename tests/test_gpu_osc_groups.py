@@ -117,3 +117,35 @@ def test_infinite_joint_state(gpu_available):
         np.testing.assert_array_equal(tau[w], want)
         np.testing.assert_array_equal(ctrl[w, acts[:n]], wctrl[:n].astype(np.float32))
     assert infinite > 20
+
+
+@pytest.mark.parametrize('config,nworld', [('c2', 21), ('c3', 21)])
+def test_osc_is_the_step_kernels_controller(gpu_available, config, nworld):
+    """mx_osc on the inputs that a control step's substep published gives that substep's torques, goal,
+    gripper and controls bit for bit (both kernels run the same 64-bit operations in the same order)."""
+    import torch
+    from libero_hip import native, scene as S
+    from libero_hip.model import Model
+    sc = S.make_scene(config, nworld, seed=2)
+    m = Model(sc)
+    d = native.DeviceData(native.DeviceModel(m), nworld)
+    rng = np.random.default_rng(22)
+    d['qpos'].copy_(torch.from_numpy(sc.init_qpos))
+    d['qvel'][:, :7].copy_(torch.from_numpy(rng.uniform(-1, 1, (nworld, 7))))
+    d['osc_gains'].copy_(torch.from_numpy(np.tile(np.r_[sc.osc['kp'], sc.osc['kd']], (nworld, 1))))
+    d['osc_q0'].copy_(torch.from_numpy(np.tile(np.asarray(sc.osc['q0'], float), (nworld, 1))))
+    d['osc_action'].copy_(torch.from_numpy(rng.uniform(-1, 1, (nworld, 7))))
+    d['body_active'].fill_(1)
+    d.forward(None, native.FLAG_BOOTSTRAP | native.FLAG_NO_CONTROL)
+    before = {k: d[k].clone() for k in ('osc_goal_pos', 'osc_goal_rot', 'osc_gripper', 'ctrl')}
+    d.control_step(1, native.FLAG_POLICY_FIRST)
+    fields = ('osc_tau', 'osc_goal_pos', 'osc_goal_rot', 'osc_gripper', 'ctrl', 'osc_rank', 'osc_error')
+    want = {k: d[k].clone() for k in fields}
+    for k, v in before.items():
+        d[k].copy_(v)
+    d['osc_tau'].zero_()
+    d.osc(native.FLAG_POLICY_FIRST)
+    torch.cuda.synchronize()
+    assert want['osc_tau'].abs().max() > 0 and not torch.equal(want['osc_goal_rot'], before['osc_goal_rot'])
+    for k in fields:
+        assert torch.equal(d[k], want[k]), k
