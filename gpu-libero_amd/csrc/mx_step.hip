@@ -89,8 +89,8 @@ enum : int { GP_MAT = 0, GP_SIZE = 9, GP_TYPE = 12, GP_MARGIN = 13, GP_GAP = 14,
 // Island sweep: block entries whose (island, row, column) a lane keeps in registers, and the words
 // per lane of the workspace route's per-substep cache of those decodes (3 per entry + 4).  The
 // workspace route is built twice, with 8 (MX_OWN default) and with 4 entries per lane: the launch
-// picks 4 for models whose contact-free island blocks take at most 192 entries (fewer registers;
-// entries beyond 64 kOwn take a slower path, so larger models keep 8).
+// picks 4 for models whose island blocks take at most 192 entries while no contact joins trees (fewer
+// registers; entries beyond 64 kOwn take a slower path, so larger models keep 8).
 #ifndef MX_OWN
 #define MX_OWN 8
 #endif
@@ -360,8 +360,7 @@ struct Ctx {
   __device__ KLayout& L() const { return params().L; }
   __device__ KImage& I() const { return params().I; }
   __device__ int w() const { return (int)blockIdx.x; }
-  // lane of the wave: the workspace route's workgroups are one wave; the LDS route's smooth kernel
-  // runs two (a mask the workspace route's stage functions, compiled out of line, would carry).
+  // Lane of the wave; a workgroup holds one wave or several on either route, so threadIdx.x is not it.
   // The workspace route recomputes it at every use, out of the optimizer's sight: per-lane
   // addresses derived from threadIdx.x are invariant across the substep loop, and hoisted out of it
   // they hold registers for the whole launch and push the stages' own values to scratch (the
@@ -1232,8 +1231,7 @@ __device__ void velocity(const Ctx& c) {
 // A pivot that is not positive and finite marks the problem failed (flag in misc[kGjFail + q]).
 struct GJProblem { int base, n, first; };
 
-template <class C>
-__device__ void gj_inverse(const C& c, const double* in, double* out, GJProblem p0, GJProblem p1,
+__device__ void gj_inverse(const Ctx& c, const double* in, double* out, GJProblem p0, GJProblem p1,
                            GJProblem p2, int nprob) {
   int lane = c.lane();
   int which = -1, n = 0, base = 0, e = 0;
@@ -1382,10 +1380,9 @@ __device__ double scaled_action(const M& m, const D& d, size_t w, int k) {
   return (x - (hi + lo) * 0.5) * (fabs(ohi - olo) / fabs(hi - lo)) + (ohi + olo) * 0.5;
 }
 
-template <bool kSplit, class C>
-__device__ void control_solve(const C& c, int policy, real* ctrl);
-template <class C>
-__device__ void control_torque(const C& c, real* ctrl);
+template <bool kSplit>
+__device__ void control_solve(const Ctx& c, int policy, real* ctrl);
+__device__ void control_torque(const Ctx& c, real* ctrl);
 
 // Controller gather (EE site Jacobian, n x n M and 6 x n J of the n = osc_ndof arm joints, q, qdot,
 // bias, EE pose/velocity in FP32 as the reference's control_drive,
@@ -1496,8 +1493,8 @@ __device__ void control_bias(const Ctx& c, bool publish) {
 // eerot, eevel) and the state in D() (goal, gripper, action, gains, q0, tau); writes tau, ctrl and,
 // at a policy substep, the goal.  (mx_osc's kernel, osc_kernel below, computes the same with eight
 // lanes per world.)
-template <bool kSplit, class C>
-__device__ void control_solve(const C& c, int policy, real* ctrl) {
+template <bool kSplit>
+__device__ void control_solve(const Ctx& c, int policy, real* ctrl) {
   KModel& m = c.m();
   const int lane = c.lane();
   int* misc = c.MISC();
@@ -1671,8 +1668,7 @@ __device__ void control_solve(const C& c, int policy, real* ctrl) {
 // force in O(dbias), clipped to the actuators' ctrl ranges (the same operations, in the same order,
 // as control_solve<false>()).  Nothing when the controller is in error (then control_solve() wrote
 // no terms).
-template <class C>
-__device__ void control_torque(const C& c, real* ctrl) {
+__device__ void control_torque(const Ctx& c, real* ctrl) {
   KModel& m = c.m();
   const int lane = c.lane(), on = m.osc_ndof;
   if (c.MISC()[kCtrlErr] != 0) return;
@@ -5143,7 +5139,7 @@ int launch(const MxModel* m, const MxData* d, const int32_t* mask, int substeps,
   if ((flags & MX_FLAG_LDS) && fits) slab = false;
   if (!slab) return launch_kernel(m, d, mask, substeps, flags, stream, obs);
   if (!have) return MX_ERR_LDS;
-  // contact-free island blocks: sum over trees of n (n + 1) / 2 = (nM + nv) / 2 packed entries
+  // the island blocks with every tree by itself: sum of n (n + 1) / 2 = (nM + nv) / 2 packed entries
   if ((m->nM + m->nv) / 2 <= 192) return mx_slab4::launch_kernel(m, d, mask, substeps, flags, stream, obs);
   return mx_slab::launch_kernel(m, d, mask, substeps, flags, stream, obs);
 }
