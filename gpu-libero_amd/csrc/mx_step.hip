@@ -5046,7 +5046,10 @@ int launch_kernel(const MxModel* m, const MxData* d, const int32_t* mask, int su
   // most.  Control step with one, two and four waves: C3 x67 5.17, 4.33, 4.00 ms; C1 x2 4.14, 3.34,
   // 3.29; the LIBERO bowl-and-plate scene x500 15.1, 14.2, 11.2; C3 x1024 (four worlds per CU) 6.21,
   // 5.38, 5.20; C3 x2048 (eight) 6.89 with one wave, 5.97 with two.  Eight waves gained 3 % on
-  // LIBERO and lost 1 to 3 % elsewhere.
+  // LIBERO and lost 1 to 3 % elsewhere.  The launch is taken to have the device to itself: batches on
+  // two streams that share CUs now run one after the other where one-wave launches ran side by side
+  // (two of C3 x1024 9.1 instead of 6.1 ms for both, two of x2048 10.8 instead of 7.7); as one batch of
+  // 2048 the former take 5.4 ms.
   const int per_cu = ncu > 0 ? (d->nworld + ncu - 1) / ncu : 16;
   int waves = m->njmax == 0 || per_cu > 8 ? 1 : (per_cu > 4 ? 2 : 4);
   while (waves > 1 && !widen_window(p.L, *m, d->nworld, ncu, waves)) waves /= 2;
