@@ -289,7 +289,8 @@ Layout make_layout(const MxModel& m) {
     // 2480 words, fifteen or sixteen worlds per CU, so that its 8192 worlds are two full rounds and not
     // two and an almost empty third (71.3 -> 59.1 ms per control step).  Elsewhere the window, which the Newton solve
     // lays itself out in too, stays the larger: in a smaller one more worlds solve on the slab's
-    // arrays, at the same precision but rounded otherwise (the LIBERO scenes' results moved).
+    // arrays, at the same precision but rounded otherwise (the LIBERO scenes' results moved; a clutter
+    // world whose solve takes between the two sizes would too, which none of those compared does).
     place(10 + 2 * it);
     if (L.win > kWindowWords) {
       place(6 + it);
